@@ -464,9 +464,9 @@ int group_shift(int gs) { return gs == 128 ? 2 : (gs == 64 ? 1 : 0); }
 
 struct Workspace {
   size_t logits, idx, w, counts, offsets, used, perm, inv, act, Y, plan_scratch;
-  size_t items_gu, items_dn;  // grouped-GEMM work items of the routed experts
+  size_t items;               // grouped-GEMM row tiles of the routed experts
   size_t x16;                 // the layer input as the GEMMs' f16 operand
-  size_t s_off, s_used, s_act, s_out, s_logit, s_items_gu, s_items_dn;
+  size_t s_off, s_used, s_act, s_out, s_logit, s_items;
   size_t xn, res;  // decoder step before the block: normalised rows, residual
   size_t total;
 };
@@ -493,8 +493,7 @@ Workspace layout(const moe_layer_desc* d, int T) {
   w.act = take(M * I * ds);
   w.Y = take(M * H * ds);
   w.plan_scratch = take(dispatch_scratch_bytes(T, (int)k, (int)E));
-  w.items_gu = take(gemm_items_bytes((int)M, (int)E, (int)I, true));
-  w.items_dn = take(gemm_items_bytes((int)M, (int)E, (int)H, false));
+  w.items = take(gemm_items_bytes((int)M, (int)E));
   w.x16 = take((size_t)T * H * 2);
   if (d->has_shared) {
     const size_t SI = (size_t)d->shared_up.n;
@@ -503,8 +502,7 @@ Workspace layout(const moe_layer_desc* d, int T) {
     w.s_act = take((size_t)T * SI * ds);
     w.s_out = take((size_t)T * H * ds);
     w.s_logit = take((size_t)T * ds);
-    w.s_items_gu = take(gemm_items_bytes(T, 1, (int)SI, true));
-    w.s_items_dn = take(gemm_items_bytes(T, 1, (int)H, false));
+    w.s_items = take(gemm_items_bytes(T, 1));
   }
   w.xn = take((size_t)T * H * ds);
   w.res = take((size_t)T * H * ds);
@@ -765,7 +763,9 @@ bool sb_words_ok(const moe_qproj& p) {
 bool gemm_ok(const moe_qproj& p, int xdt, int M, const void* out = nullptr) {
   const int slots = std::min(p.n_experts, M);
   // activation rows are addressed with 32-bit byte offsets
-  const bool fits = (size_t)M * (size_t)p.k * 2 < (1ull << 32);
+  // (and an expert's weight rows, up to a block's past the last one)
+  const bool fits = (size_t)M * (size_t)p.k * 2 < (1ull << 32) &&
+                    ((size_t)p.n + 256) * ((size_t)p.k * p.bits / 8) < (1ull << 32);
   return xdt != MOE_F32 && p.k % 64 == 0 && p.n % 8 == 0 && p.n_experts <= 1024 && fits && sb_words_ok(p) &&
          M >= (p.n_experts >= kGemmManyExperts ? kGemmMinRowsMany : kGemmMinRows) * slots &&
          (reinterpret_cast<uintptr_t>(out) & 15) == 0;
@@ -815,8 +815,9 @@ moe_status run_gemm(const moe_qproj& p0, const moe_qproj* p1, const void* x, int
   a.alpha = alpha;
   a.limit = limit;
   const bool gu = p1 != nullptr;
-  const long items_max = gemm_max_items(M, p0.n_experts, p0.n, gu);
-  const int grid = (int)((items_max + 7) / 8 * 8);  // a multiple of the 8 XCDs
+  a.col_blocks = gemm_col_blocks(p0.n, gu);
+  const long most = gemm_max_tiles(M, p0.n_experts) * a.col_blocks;
+  const int grid = (int)((most + 7) / 8 * 8);  // a multiple of the 8 XCDs
   MOE_HIP(launch_gemm(p0.bits, xdt, p0.sb_dtype, gu, a, grid, st, ev),
           "grouped GEMM launch");
   return MOE_OK;
@@ -977,7 +978,7 @@ extern "C" moe_status moe_mxfp4_to_affine(const uint32_t* packed, const uint8_t*
 extern "C" size_t moe_expert_matmul_workspace_bytes(const moe_qproj* p, int32_t a_dtype, int32_t M) {
   if (!p || M <= 0 || validate_qproj_named(p, "expert_matmul") != MOE_OK || !dt_ok(a_dtype)) return 0;
   size_t bytes = align_up((size_t)(p->n_experts + 1) * 4, 256) +
-                 align_up(gemm_items_bytes(M, p->n_experts, p->n, false), 256);
+                 align_up(gemm_items_bytes(M, p->n_experts), 256);
   if (a_dtype == MOE_BF16) bytes += align_up((size_t)M * p->k * 2, 256);
   return bytes;
 }
@@ -1000,11 +1001,11 @@ extern "C" moe_status moe_expert_matmul(const moe_qproj* p, const void* a, int32
     char* wsc = reinterpret_cast<char*>(workspace);
     const size_t items_at = align_up((size_t)(p->n_experts + 1) * 4, 256);
     uint32_t* items = reinterpret_cast<uint32_t*>(wsc + items_at);
-    MOE_HIP(launch_gemm_items(offsets, p->n_experts, p->n, false, items, 0, false, nullptr, stream),
+    MOE_HIP(launch_gemm_items(offsets, p->n_experts, items, stream),
             "GEMM work list launch");
     const void* a16 = a;
     if (a_dtype == MOE_BF16) {  // the GEMM's f16 operand: bf16 rows scaled by 2^-kA16Shift
-      void* x16 = wsc + items_at + align_up(gemm_items_bytes(M, p->n_experts, p->n, false), 256);
+      void* x16 = wsc + items_at + align_up(gemm_items_bytes(M, p->n_experts), 256);
       const int64_t rows = perm ? (M + top_k - 1) / top_k : M;
       MOE_HIP(launch_to_a16(a, x16, rows * p->k, stream), "f16 operand launch");
       a16 = x16;
@@ -1235,15 +1236,13 @@ moe_status shared_expert(const moe_layer_desc* d, const void* x, const void* x16
   const moe_qproj* p1 = gated ? &d->shared_up : nullptr;
   if (shared_gemm(d, T)) {
     // many tokens through one expert: the matrix-core path
-    MOE_HIP(launch_gemm_items(at<uint32_t>(ws, w.s_off), 1, p0.n, p1 != nullptr,
-                              at<uint32_t>(ws, w.s_items_gu), d->hidden, false,
-                              at<uint32_t>(ws, w.s_items_dn), st),
+    MOE_HIP(launch_gemm_items(at<uint32_t>(ws, w.s_off), 1, at<uint32_t>(ws, w.s_items), st),
             "shared GEMM work list launch");
     MOE_TRY(run_gemm(p0, p1, x16, xdt, true, nullptr, 1, at<uint32_t>(ws, w.s_off),
-                     at<uint32_t>(ws, w.s_items_gu), T, at<void>(ws, w.s_act), d->activation,
+                     at<uint32_t>(ws, w.s_items), T, at<void>(ws, w.s_act), d->activation,
                      d->act_alpha, d->act_limit, st));
     MOE_TRY(run_gemm(d->shared_down, nullptr, at<void>(ws, w.s_act), xdt, false, nullptr, 1,
-                     at<uint32_t>(ws, w.s_off), at<uint32_t>(ws, w.s_items_dn), T,
+                     at<uint32_t>(ws, w.s_off), at<uint32_t>(ws, w.s_items), T,
                      at<void>(ws, w.s_out), 0, 0.f, 0.f, st));
   } else {
     MOE_TRY(run_gemv(p0, p1, x, xdt, nullptr, 1, at<uint32_t>(ws, w.s_off),
@@ -1597,9 +1596,7 @@ moe_status layer_forward(const moe_layer_desc* d, const void* x, const void* rx,
     const bool gated = d->activation != MOE_ACT_RELU2;
     const moe_qproj& p0 = gated ? d->gate : d->up;
     const moe_qproj* p1 = gated ? &d->up : nullptr;
-    // the GEMM work lists, written by the plan's last launch when it can
-    const GemmItemsReq ireq{p0.n, p1 != nullptr, at<uint32_t>(ws, w.items_gu),
-                            H,    false,         at<uint32_t>(ws, w.items_dn)};
+    // the GEMM's row tiles, written by the plan's last launch when it can
     bool items_done = false;
     // 2. selection + dispatch plan (MoELayer.swift:706-792): one launch for a
     //    small batch, else the top-k and plan kernels (past 8 tokens the GEMM
@@ -1619,18 +1616,17 @@ moe_status layer_forward(const moe_layer_desc* d, const void* x, const void* rx,
                                    at<uint32_t>(ws, w.offsets), at<uint32_t>(ws, w.perm),
                                    at<uint32_t>(ws, w.inv), at<uint32_t>(ws, w.used),
                                    at<void>(ws, w.plan_scratch), dispatch_scratch_bytes(T, k, E),
-                                   st, gemm ? &ireq : nullptr, &items_done),
+                                   st, gemm ? at<uint32_t>(ws, w.items) : nullptr, &items_done),
               "dispatch plan launch");
     }
     const int slots = std::min(E, M);
     // 3. gate/up + activation over the plan (MoELayer.swift:883-893)
     if (gemm) {
       if (!items_done)
-        MOE_HIP(launch_gemm_items(at<uint32_t>(ws, w.offsets), E, ireq.N0, ireq.gateup0,
-                                  ireq.items0, ireq.N1, ireq.gateup1, ireq.items1, st),
+        MOE_HIP(launch_gemm_items(at<uint32_t>(ws, w.offsets), E, at<uint32_t>(ws, w.items), st),
                 "GEMM work list launch");
       MOE_TRY(run_gemm(p0, p1, x16, xdt, true, at<uint32_t>(ws, w.perm), k,
-                       at<uint32_t>(ws, w.offsets), at<uint32_t>(ws, w.items_gu), M,
+                       at<uint32_t>(ws, w.offsets), at<uint32_t>(ws, w.items), M,
                        at<void>(ws, w.act), d->activation, d->act_alpha, d->act_limit, st, kev(0)));
     } else {
       MOE_TRY(run_gemv(p0, p1, x, xdt, at<uint32_t>(ws, w.perm), k,
@@ -1641,7 +1637,7 @@ moe_status layer_forward(const moe_layer_desc* d, const void* x, const void* rx,
     // 4. down projection, then the weighted combine (MoELayer.swift:899-939)
     if (gemm) {
       MOE_TRY(run_gemm(d->down, nullptr, at<void>(ws, w.act), xdt, false, nullptr, 1,
-                       at<uint32_t>(ws, w.offsets), at<uint32_t>(ws, w.items_dn), M,
+                       at<uint32_t>(ws, w.offsets), at<uint32_t>(ws, w.items), M,
                        at<void>(ws, w.Y), 0, 0.f, 0.f, st, kev(1)));
     } else {
       MOE_TRY(run_gemv(d->down, nullptr, at<void>(ws, w.act), xdt, nullptr, 1,

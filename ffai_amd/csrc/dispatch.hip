@@ -357,130 +357,63 @@ size_t dispatch_scratch_bytes(int T, int k, int E) {
   return (size_t)(nchunks * E * 4);
 }
 
-constexpr int kItemBlocks = 8;  // blocks writing the GEMM work items
-
-struct ItemCols {
-  int nb[2][kGemmShapes];  // column blocks per tile shape, for each of the two lists
-};
-
-// Work items of the grouped GEMM over an expert-sorted plan (the list format
-// is described at launch_gemm_items). Thread t counts the items of experts
-// t * EPT .. + EPT; a block scan gives every expert's first item (in LDS),
-// the same in every block; then the threads of all blocks write items in a
-// strided loop, each finding its expert by a binary search over those starts.
-__device__ void gemm_items_body(const uint32_t* __restrict__ offsets, int E, const ItemCols& ic,
-                                uint32_t* __restrict__ items0, uint32_t* __restrict__ items1,
-                                int blk, int nblk) {
-  __shared__ uint32_t scan[2][kPlanThreads];
-  __shared__ uint32_t start[2][kPlanMaxE + 1];  // first item of each expert, per list
-  __shared__ uint32_t first_pos[kPlanMaxE], rows_of[kPlanMaxE];
+// Row tiles of the grouped GEMM over an expert-sorted plan (the list format is
+// described at launch_gemm_items): thread t counts the tiles of experts
+// t * EPT .. + EPT, a block scan gives each expert's first tile, and the
+// thread writes its experts' tiles (a tile holds up to kGemmTileRows rows, so
+// an expert has few).
+__device__ void gemm_items_body(const uint32_t* __restrict__ offsets, int E,
+                                uint32_t* __restrict__ items) {
+  __shared__ uint32_t wsum[kPlanThreads / 64];
   constexpr int EPT = kPlanMaxE / kPlanThreads;  // experts per thread
-  const int t = threadIdx.x;
-  uint32_t cnt[2][EPT], tot0 = 0, tot1 = 0;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  uint32_t first[EPT], rows[EPT], tot = 0;
 #pragma unroll
   for (int j = 0; j < EPT; j++) {
     const int e = t * EPT + j;
-    uint32_t rows = 0, first = 0;
-    if (e < E) {
-      first = offsets[e];
-      rows = offsets[e + 1] - first;
-      first_pos[e] = first;
-      rows_of[e] = rows;
-    }
-    const uint32_t full = rows / 256u, rem = rows % 256u;
-    // the remainder takes the smallest shape that holds it
-    const int rs = gemm_shape_for((int)rem);
-    cnt[0][j] = full * (uint32_t)ic.nb[0][0] + (rem ? (uint32_t)ic.nb[0][rs] : 0u);
-    cnt[1][j] = full * (uint32_t)ic.nb[1][0] + (rem ? (uint32_t)ic.nb[1][rs] : 0u);
-    tot0 += cnt[0][j];
-    tot1 += cnt[1][j];
+    first[j] = e < E ? offsets[e] : 0u;
+    rows[j] = e < E ? offsets[e + 1] - first[j] : 0u;
+    tot += (rows[j] + kGemmTileRows - 1u) / kGemmTileRows;
   }
-  scan[0][t] = tot0;
-  scan[1][t] = tot1;
+  const uint32_t s = wave_scan_u32(tot);
+  if (lane == 63) wsum[wave] = s;
   __syncthreads();
-  for (int off = 1; off < kPlanThreads; off <<= 1) {
-    const uint32_t v0 = t >= off ? scan[0][t - off] : 0u;
-    const uint32_t v1 = t >= off ? scan[1][t - off] : 0u;
-    __syncthreads();
-    scan[0][t] += v0;
-    scan[1][t] += v1;
-    __syncthreads();
+  uint32_t at = s - tot, all = 0;
+#pragma unroll
+  for (int w = 0; w < kPlanThreads / 64; w++) {
+    at += w < wave ? wsum[w] : 0u;
+    all += wsum[w];
   }
-  uint32_t b0 = scan[0][t] - tot0, b1 = scan[1][t] - tot1;
+  if (t == 0) items[0] = all;
 #pragma unroll
   for (int j = 0; j < EPT; j++) {
-    const int e = t * EPT + j;
-    if (e < E) {
-      start[0][e] = b0;
-      start[1][e] = b1;
-    }
-    b0 += cnt[0][j];
-    b1 += cnt[1][j];
-  }
-  const uint32_t n[2] = {scan[0][kPlanThreads - 1], scan[1][kPlanThreads - 1]};
-  if (t == 0) {
-    start[0][E] = n[0];
-    start[1][E] = n[1];
-    if (blk == 0) {
-      items0[0] = n[0];
-      if (items1) items1[0] = n[1];
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int l = 0; l < 2; l++) {
-    uint32_t* items = l ? items1 : items0;
-    if (!items) continue;
-    const uint32_t nb0 = (uint32_t)ic.nb[l][0];
-    for (uint32_t i = (uint32_t)blk * kPlanThreads + (uint32_t)t; i < n[l];
-         i += (uint32_t)nblk * kPlanThreads) {
-      // the last expert whose first item is at or before i (experts without
-      // items share their start with the next one)
-      int lo = 0, hi = E - 1;
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (start[l][mid] <= i) lo = mid;
-        else hi = mid - 1;
-      }
-      const uint32_t e = (uint32_t)lo, k = i - start[l][lo];
-      const uint32_t rows = rows_of[e], full = rows / 256u;
-      uint32_t tile, b, shape;
-      if (k < full * nb0) {
-        tile = k / nb0;
-        b = k - tile * nb0;
-        shape = 0u;
-      } else {
-        const uint32_t rem = rows % 256u;
-        tile = full;
-        b = k - full * nb0;
-        shape = (uint32_t)gemm_shape_for((int)rem);
-      }
-      uint32_t* it = items + 4 + 4 * i;
-      it[0] = e | (shape << 30);
-      it[1] = first_pos[e] + tile * 256u;
-      it[2] = b;
-      it[3] = first_pos[e] + rows;
+    for (uint32_t r = 0; r < rows[j]; r += kGemmTileRows, at++) {
+      items[4 + 2 * at] = (uint32_t)(t * EPT + j);
+      items[5 + 2 * at] = (first[j] + r) | ((min(rows[j] - r, (uint32_t)kGemmTileRows) - 1u) << 25);
     }
   }
 }
 
 __global__ __launch_bounds__(kPlanThreads) void gemm_items_kernel(
-    const uint32_t* __restrict__ offsets, int E, const ItemCols ic, uint32_t* __restrict__ items0,
-    uint32_t* __restrict__ items1) {
-  gemm_items_body(offsets, E, ic, items0, items1, (int)blockIdx.x, (int)gridDim.x);
+    const uint32_t* __restrict__ offsets, int E, uint32_t* __restrict__ items) {
+  gemm_items_body(offsets, E, items);
 }
 
-// Multi-block pass 3 with the grouped GEMM's work items: each block scatters
-// its chunk as plan_scatter_kernel does, then writes a strided share of the
-// items as gemm_items_kernel does (they need only the offsets, which the
-// scan pass wrote). One launch fewer per prefill step.
+// Multi-block pass 3 with the grouped GEMM's row tiles: each block scatters
+// its chunk as plan_scatter_kernel does, and one more block writes the tiles
+// (they need only the offsets, which the scan pass wrote). One launch fewer
+// per prefill step.
 __global__ __launch_bounds__(kPlanThreads) void plan_scatter_items_kernel(
     const uint32_t* __restrict__ idx, int M, int E, const uint32_t* __restrict__ hist,
-    uint32_t* perm, uint32_t* inv, const uint32_t* __restrict__ offsets, const ItemCols ic,
-    uint32_t* __restrict__ items0, uint32_t* __restrict__ items1) {
+    uint32_t* perm, uint32_t* inv, const uint32_t* __restrict__ offsets,
+    uint32_t* __restrict__ items) {
   __shared__ uint32_t cursor[kPlanMaxE];
   constexpr int PER = kChunk / kPlanThreads;
   const int tid = threadIdx.x, c = blockIdx.x;
+  if (c == (int)gridDim.x - 1) {
+    gemm_items_body(offsets, E, items);
+    return;
+  }
   const int begin = c * kChunk, end = min(M, begin + kChunk);
   uint32_t ev[PER];  // the chunk's ids, all loads in flight at once
 #pragma unroll
@@ -491,22 +424,12 @@ __global__ __launch_bounds__(kPlanThreads) void plan_scatter_items_kernel(
   for (int e = tid; e < E; e += kPlanThreads) cursor[e] = hist[(size_t)c * E + e];
   __syncthreads();
   stable_scatter_held<kPlanThreads, PER>(ev, begin, end - begin, E, id_bits(E), cursor, perm, inv);
-  gemm_items_body(offsets, E, ic, items0, items1, c, (int)gridDim.x);
-}
-
-static ItemCols item_cols(int N0, bool gateup0, int N1, bool gateup1, bool two) {
-  ItemCols ic{};
-  for (int sh = 0; sh < kGemmShapes; sh++) {
-    ic.nb[0][sh] = (N0 + gemm_cols(sh, gateup0) - 1) / gemm_cols(sh, gateup0);
-    ic.nb[1][sh] = two ? (N1 + gemm_cols(sh, gateup1) - 1) / gemm_cols(sh, gateup1) : 0;
-  }
-  return ic;
 }
 
 hipError_t launch_dispatch_plan(const uint32_t* idx, int T, int k, int E, uint32_t* counts,
                                 uint32_t* offsets, uint32_t* perm, uint32_t* inv_perm,
                                 uint32_t* used, void* scratch, size_t scratch_bytes,
-                                hipStream_t st, const GemmItemsReq* items, bool* items_done) {
+                                hipStream_t st, uint32_t* items, bool* items_done) {
   if (items_done) *items_done = false;
   const int M = T * k;
   if (E > kPlanMaxE) return hipErrorInvalidValue;
@@ -522,10 +445,8 @@ hipError_t launch_dispatch_plan(const uint32_t* idx, int T, int k, int E, uint32
   hipLaunchKernelGGL(plan_scan_kernel, dim3(1), dim3(kPlanThreads), 0, st, nchunks, E, hist,
                      counts, offsets, used);
   if (items) {
-    const ItemCols ic = item_cols(items->N0, items->gateup0, items->N1, items->gateup1,
-                                  items->items1 != nullptr);
-    hipLaunchKernelGGL(plan_scatter_items_kernel, dim3(nchunks), dim3(kPlanThreads), 0, st, idx,
-                       M, E, hist, perm, inv_perm, offsets, ic, items->items0, items->items1);
+    hipLaunchKernelGGL(plan_scatter_items_kernel, dim3(nchunks + 1), dim3(kPlanThreads), 0, st, idx,
+                       M, E, hist, perm, inv_perm, offsets, items);
     if (items_done) *items_done = true;
   } else {
     hipLaunchKernelGGL(plan_scatter_kernel, dim3(nchunks), dim3(kPlanThreads), 0, st, idx, M, E,
@@ -534,15 +455,9 @@ hipError_t launch_dispatch_plan(const uint32_t* idx, int T, int k, int E, uint32
   return hipGetLastError();
 }
 
-hipError_t launch_gemm_items(const uint32_t* offsets, int E, int N0, bool gateup0,
-                             uint32_t* items0, int N1, bool gateup1, uint32_t* items1,
-                             hipStream_t st) {
+hipError_t launch_gemm_items(const uint32_t* offsets, int E, uint32_t* items, hipStream_t st) {
   if (E > kPlanMaxE) return hipErrorInvalidValue;
-  const ItemCols ic = item_cols(N0, gateup0, N1, gateup1, items1 != nullptr);
-  // every block scans the experts' item counts (cheap) and writes a strided
-  // share of the items
-  hipLaunchKernelGGL(gemm_items_kernel, dim3(kItemBlocks), dim3(kPlanThreads), 0, st, offsets, E, ic, items0,
-                     items1);
+  hipLaunchKernelGGL(gemm_items_kernel, dim3(1), dim3(kPlanThreads), 0, st, offsets, E, items);
   return hipGetLastError();
 }
 

@@ -191,22 +191,13 @@ hipError_t launch_router_q(int bits, const void* x, int xdt, int T, int H, const
 hipError_t launch_route_plan(const void* logits, int dt, int T, int E, int k, const RouteOpts& ro,
                              uint32_t* idx, float* w, uint32_t* counts, uint32_t* offsets,
                              uint32_t* perm, uint32_t* inv, uint32_t* used, hipStream_t st);
-// The grouped GEMM's work items (launch_gemm_items arguments) to be written
-// by the plan's last launch.
-struct GemmItemsReq {
-  int N0;
-  bool gateup0;
-  uint32_t* items0;
-  int N1;
-  bool gateup1;
-  uint32_t* items1;  // nullptr: one list
-};
-// With `items`, a multi-block plan also writes the GEMM work items (then
-// *items_done is set; a one-workgroup plan leaves them to launch_gemm_items).
+// With `items`, a multi-block plan also writes the GEMM's row tiles there
+// (then *items_done is set; a one-workgroup plan leaves them to
+// launch_gemm_items).
 hipError_t launch_dispatch_plan(const uint32_t* idx, int T, int k, int E, uint32_t* counts,
                                 uint32_t* offsets, uint32_t* perm, uint32_t* inv_perm,
                                 uint32_t* used, void* scratch, size_t scratch_bytes,
-                                hipStream_t st, const GemmItemsReq* items = nullptr,
+                                hipStream_t st, uint32_t* items = nullptr,
                                 bool* items_done = nullptr);
 size_t dispatch_scratch_bytes(int T, int k, int E);
 // Fills offsets {0, M}, used {1, 0} for a single-expert identity plan.
@@ -257,7 +248,8 @@ struct GemmArgs {
   const uint32_t* perm;      // nullable: row(p) = perm[p] / topk, else p
   int topk;
   const uint32_t* offsets;   // [E+1] CSR over sorted positions
-  const uint32_t* items;     // work items (launch_gemm_items)
+  const uint32_t* items;     // row tiles (launch_gemm_items)
+  int col_blocks;            // gemm_col_blocks(N, pair)
   void* out;                 // [M, N]
   int N, K, gsh;
   int sb_bf16;               // scales / biases stored as bf16 (else f16)
@@ -266,39 +258,25 @@ struct GemmArgs {
   int act;
   float alpha, limit;
 };
-// Block shapes (activation rows x weight rows per block, 8 waves): an
-// expert's rows go in 256-row tiles, and its last tile is the smallest shape
-// that holds what is left.
-constexpr int kGemmShapes = 3;
-constexpr int kGemmShapeRows[kGemmShapes] = {256, 128, 64};
-constexpr int kGemmShapeWRows[kGemmShapes] = {256, 256, 256};
-__host__ __device__ inline int gemm_shape_for(int rows) {
-  return rows > 128 ? 0 : (rows > 64 ? 1 : 2);
+// A block takes a tile of up to kGemmTileRows of an expert's rows and
+// kGemmTileWRows weight rows (half gate, half up rows for a pair).
+constexpr int kGemmTileRows = 96;
+constexpr int kGemmTileWRows = 128;
+// Column blocks per row tile.
+inline int gemm_col_blocks(int N, bool gateup) {
+  const int cols = gateup ? kGemmTileWRows / 2 : kGemmTileWRows;
+  return (N + cols - 1) / cols;
 }
-// Output columns per block: half the weight rows for a gate/up pair.
-inline int gemm_cols(int shape, bool gateup) {
-  return gateup ? kGemmShapeWRows[shape] / 2 : kGemmShapeWRows[shape];
-}
-// Upper bound on the work items of a plan of M rows over E experts (shapes
-// 0 and 1 have the most column blocks).
-inline long gemm_max_items(int M, int E, int N, bool gateup) {
-  const long tiles = (M + 255) / 256 + (long)E;
-  return tiles * ((N + gemm_cols(0, gateup) - 1) / gemm_cols(0, gateup));
-}
-inline size_t gemm_items_bytes(int M, int E, int N, bool gateup) {
-  return (size_t)(4 + 4 * gemm_max_items(M, E, N, gateup)) * 4;
-}
-// items[0] = count (items[1..3] unused), then per item, 16-byte aligned,
-// {expert | shape << 30, first sorted position, column block, end of the
-// expert's positions}: experts ascending, an expert's row tiles in order, a
-// tile's column blocks in order (neighbouring items share activation rows).
-// Writes the list for (N0, gateup0) into items0 and, when items1 is
-// non-NULL, the list for (N1, gateup1) over the same tiles into items1.
-hipError_t launch_gemm_items(const uint32_t* offsets, int E, int N0, bool gateup0,
-                             uint32_t* items0, int N1, bool gateup1, uint32_t* items1,
-                             hipStream_t st);
-// grid: 8 * ceil(gemm_max_items / 8) blocks (items are split evenly over the
-// XCDs at run time; blocks without an item return at once).
+// Upper bound on the row tiles of a plan of M rows over E experts.
+inline long gemm_max_tiles(int M, int E) { return M / kGemmTileRows + (long)E; }
+inline size_t gemm_items_bytes(int M, int E) { return (size_t)(4 + 2 * gemm_max_tiles(M, E)) * 4; }
+// The row tiles of a plan: items[0] = count (items[1..3] unused), then 8
+// bytes per tile: expert, first sorted position | (rows - 1) << 25 (at most
+// 2^25 positions): experts ascending, an expert's tiles in order.
+hipError_t launch_gemm_items(const uint32_t* offsets, int E, uint32_t* items, hipStream_t st);
+// grid: 8 * ceil(gemm_max_tiles * col_blocks / 8) blocks (the (tile, column
+// block) pairs are split evenly over the XCDs at run time; blocks without one
+// return at once).
 hipError_t launch_gemm(int bits, int xdt, int sbdt, bool gateup, const GemmArgs& a, int grid,
                        hipStream_t st, KEvents ev = {});
 // Elementwise bf16 -> f16 * 2^-kA16Shift (saturating), n a multiple of 8,

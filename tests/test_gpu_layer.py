@@ -290,6 +290,50 @@ def test_expert_matmul_mfma(bits, dt, sb, gs, gather):
     check_close(to_numpy_f32(out), ref, dt, f"mfma expert_matmul bits={bits} gs={gs}")
 
 
+@pytest.mark.parametrize("bits,dt,sb,gs,K", [
+    (4, BF16, F16, 64, 64),     # one half chunk
+    (4, BF16, BF16, 64, 192),   # an odd number of groups per row, a half last chunk
+    (3, BF16, BF16, 64, 960),   # odd groups, a half chunk after whole trips
+    (4, F16, F16, 32, 576),     # two-chunk scale segments, half last chunk
+    (2, F16, F16, 128, 640),    # odd groups of 128
+    (4, BF16, F16, 128, 1152),
+    (6, BF16, BF16, 64, 832),
+    (8, F16, F16, 32, 320),
+    (5, F16, BF16, 64, 448),
+])
+@pytest.mark.parametrize("counts", [(1, 96, 97), (33, 0, 65), (32, 64, 193)])
+@pytest.mark.parametrize("N", [8, 136])
+def test_expert_matmul_tile_edges(bits, dt, sb, gs, K, counts, N):
+    """Row tiles of 32, 64 and 96 rows and one more, one row, no row; one
+    group of 8 output columns and a column block plus one; K with and without
+    a half last chunk, odd group counts. Tolerance: the layer bar, as
+    test_expert_matmul_mfma (the weights are rounded once to f16)."""
+    from moe_spec import gen_qproj
+    rng = np.random.default_rng(bits * 1000 + K + N)
+    E, M = len(counts), int(sum(counts))
+    f = 15.0 / (2 ** bits - 1)
+    p = gen_qproj(rng, E, N, K, bits, gs, sb, s_range=(0.005 * f, 0.02 * f))
+    experts = np.repeat(np.arange(E), counts).astype(np.uint32)
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32)
+    a = store(rng.normal(0, 1, (M, K)), dt)
+    lib = _lib.load()
+    q = _lib.QProj(0, 0, 0, None, bits, gs, sb, N, K, E)
+    wt, st, bt = to_torch(p.weight.view(np.int32)), to_torch(p.scales), to_torch(p.biases)
+    q.weight, q.scales, q.biases = wt.data_ptr(), st.data_ptr(), bt.data_ptr()
+    at = to_torch(a)
+    out = torch.empty(M, N, dtype=at.dtype, device="cuda")
+    wsb = lib.moe_expert_matmul_workspace_bytes(C.byref(q), dt, M)
+    ws = torch.empty(wsb, dtype=torch.uint8, device="cuda")
+    offt = to_torch(offsets.view(np.int32))
+    for _ in range(3):  # repeated calls give the same bits
+        check(lib.moe_expert_matmul(C.byref(q), _p(at), dt, None, 1, M, _p(offt), _p(out), _p(ws), wsb,
+                                    _stream()))
+        torch.cuda.synchronize()
+        got = to_numpy_f32(out)
+        ref = orc.round_dt(orc.qgemm_rows(p, load(a, dt), experts), dt)
+        check_close(got, ref, dt, f"tile edges bits={bits} gs={gs} K={K} rows={counts} N={N}")
+
+
 def test_gemm_operand_range_bf16():
     """The matrix-core path feeds a bf16 input to the matrix cores as f16
     values x 2^-8, converted to nearest: a row element at 2^25 (beyond
