@@ -45,6 +45,7 @@ hipError_t launch_mma_b3(int, int, bool, const GemvArgs&, int, hipStream_t, KEve
 hipError_t launch_mma_b4(int, int, bool, const GemvArgs&, int, hipStream_t, KEvents);
 hipError_t launch_mma_b5(int, int, bool, const GemvArgs&, int, hipStream_t, KEvents);
 hipError_t launch_mma_b6(int, int, bool, const GemvArgs&, int, hipStream_t, KEvents);
+hipError_t launch_mma_b8(int, int, bool, const GemvArgs&, int, hipStream_t, KEvents);
 
 static hipError_t launch_mma(int bits, int xdt, int sbdt, bool gateup, const GemvArgs& a,
                              int grid, hipStream_t st, KEvents ev) {
@@ -54,6 +55,7 @@ static hipError_t launch_mma(int bits, int xdt, int sbdt, bool gateup, const Gem
     case 4: return launch_mma_b4(xdt, sbdt, gateup, a, grid, st, ev);
     case 5: return launch_mma_b5(xdt, sbdt, gateup, a, grid, st, ev);
     case 6: return launch_mma_b6(xdt, sbdt, gateup, a, grid, st, ev);
+    case 8: return launch_mma_b8(xdt, sbdt, gateup, a, grid, st, ev);
     default: return hipErrorInvalidValue;
   }
 }
@@ -555,12 +557,18 @@ constexpr int kMmaMinRowsPair10 = 10;
 constexpr int kMmaMinRowsSingle10 = 18;
 constexpr int kMmaMinRowsOther10 = 20;
 constexpr int kMmaMinRowsSingleExpert10 = 160;
+// Tenths of a row per used expert from which the matrix-core GEMV takes 32
+// activation rows per pass instead of 16 (µs per layer step, 16 / 32 rows per
+// pass: 15.6 rows on 128 experts 342 / 327, 16 and 23 rows on 32 large experts
+// 226 / 199 and 276 / 225; at 10 and 14 rows on 128 experts 126 / 150 and
+// 150 / 155).
+constexpr int kMmaWideRows10 = 150;
 
-// gemv_mma_kernel applies: 2- to 6-bit codes (exact with the magic offset in
-// either 16-bit type), 16-bit activations at 16-byte aligned rows, and
+// gemv_mma_kernel applies: codes of one width (every width is exact in either
+// 16-bit type), 16-bit activations at 16-byte aligned rows, and
 // expert-local byte offsets below 2^31.
 bool mma_ok(const moe_qproj& p0, const moe_qproj* p1, bool x_aligned, int xdt) {
-  if (p0.bits < 2 || p0.bits > 6 || (p1 && p1->bits != p0.bits)) return false;
+  if (p1 && p1->bits != p0.bits) return false;
   if (xdt == MOE_F32 || p0.sb_dtype == MOE_F32 || !x_aligned) return false;
   return ((size_t)p0.n + 64) * ((size_t)p0.k * p0.bits / 8) < (1ull << 31);
 }
@@ -651,12 +659,12 @@ void run_multi(const moe_qproj& p0, const moe_qproj* p1, const void* x, int xdt,
   *status = hip_check(err, "grouped GEMV launch");
 }
 
-// gemv_mma_kernel (matrix cores) for 2- to 6-bit weights and 16-bit
+// gemv_mma_kernel (matrix cores) for 16-bit
 // activations: 32 rows of a gate/up pair or 64 rows of one projection per
 // block, 16 activation rows per pass. The caller has checked mma_ok.
 void run_mma(const moe_qproj& p0, const moe_qproj* p1, const void* x, int xdt,
              const uint32_t* perm, int topk, const uint32_t* offsets, const uint32_t* used, int slots,
-             int x_rows, void* out, int act, float alpha, float limit, hipStream_t st, KEvents ev,
+             int M, int x_rows, void* out, int act, float alpha, float limit, hipStream_t st, KEvents ev,
              moe_status* status) {
   const int rows_per_block = p1 ? 32 : 64;
   const int row_blocks = (p0.n + rows_per_block - 1) / rows_per_block;
@@ -678,6 +686,7 @@ void run_mma(const moe_qproj& p0, const moe_qproj* p1, const void* x, int xdt,
   a.alpha = alpha;
   a.limit = limit;
   a.x_rows = x_rows;
+  a.tok_chunk = 10L * M >= (long)kMmaWideRows10 * std::max(1, slots) ? 32 : 16;
   *status = hip_check(launch_mma(p0.bits, xdt, p0.sb_dtype, p1 != nullptr, a, slots * row_blocks, st, ev),
                       "grouped GEMV launch");
 }
@@ -694,7 +703,7 @@ moe_status run_gemv(const moe_qproj& p0, const moe_qproj* p1, const void* x, int
     moe_status status = MOE_OK;
     // the activation rows: one per token on the gather path (M = T topk)
     const int x_rows = perm ? (M + topk - 1) / topk : M;
-    run_mma(p0, p1, x, xdt, perm, topk, offsets, used, slots, x_rows, out, act, alpha, limit, st,
+    run_mma(p0, p1, x, xdt, perm, topk, offsets, used, slots, M, x_rows, out, act, alpha, limit, st,
             ev, &status);
     return status;
   }

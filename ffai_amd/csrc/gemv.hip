@@ -377,10 +377,9 @@ __global__ __launch_bounds__(256, 2) void gemv_multi_kernel(const GemvArgs a) {
 #define MOE_CAT2(a, b) a##b
 #define MOE_CAT(a, b) MOE_CAT2(a, b)
 
-#if MOE_BITS <= 6
 // ---------------------------------------------------------------------------
-// grouped GEMV for a few rows per expert on the matrix cores (4-bit weights,
-// 16-bit activations)
+// grouped GEMV for a few rows per expert on the matrix cores (16-bit
+// activations)
 //
 // Block (slot, rb): expert used[1 + slot] and 64 LDS weight rows (a gate/up
 // pair: 32 rows of each; else 64 rows of one projection); the expert's
@@ -395,10 +394,20 @@ __global__ __launch_bounds__(256, 2) void gemv_multi_kernel(const GemvArgs a) {
 // [8 kb BITS, +8 BITS) of the unit's BITS words; for 4 bits, word kb), whose
 // pairs (j, j + 4) match the activations' pair order, and
 // quad kb of activation row r; it ends with rows 4 kb + i of output column r.
-// K runs in chunks of 8 units through double-buffered LDS: per chunk the
-// block copies 64 rows x 8 units of codes (BITS words each), their 16-bit
-// scale/bias pairs and 16 rows x 8 units of activations (permuted to pair
-// order), with global loads two chunks ahead of the MFMAs.
+// K runs in chunks of 8 units (8 bits: 4) through double-buffered LDS: per
+// chunk the block copies 64 rows x 8 units of codes (BITS words each), their
+// 16-bit scale/bias pairs and 16 rows x 8 units of activations (permuted to
+// pair order), with global loads two chunks ahead of the MFMAs.
+// 8-bit codes: 1024 + code is exact in f16, and bf16 holds 0..255 exactly as
+// they are (MAGIC 0). gemv_multi_kernel, which 8-bit weights took before, is
+// bound by its unpacking there (64 experts of 1024 x 384, f16, groups of 32,
+// 48 tokens: gate/up 40.9 -> 16.9 us, down 20.3 -> 10.6, layer step 80 -> 49).
+// From 15 rows per used expert a pass takes 32 rows (TT = 2): most experts
+// then exceed 16 rows, and each further pass streams and unpacks the weights
+// again (32 experts of 2880 x 2880, 128 / 184 tokens 226 -> 199, 276 -> 225 us
+// per layer step; 128 experts with 15.6 rows 342 -> 327). Below, its LDS
+// (three blocks per CU instead of four) costs more: 128 experts of 2048 x 768
+// at 10 rows 126 -> 150 us.
 // ---------------------------------------------------------------------------
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -419,9 +428,10 @@ template <> struct Mma16<f16_t> {
   }
 };
 
-constexpr int kMmaU = 8;      // units per K chunk
+// Units per K chunk: a 128-byte line of a weight row at 4 and 8 bits (half the
+// LDS per 8-bit chunk keeps five blocks per CU instead of two).
+template <int BITS> constexpr int kMmaUnits = BITS == 8 ? 4 : 8;
 constexpr int kMmaRows = 64;  // LDS weight rows per block
-constexpr int kMmaTok = 16;   // activation rows per pass
 
 // Codes of 8-value block kb of a unit as four magic-offset pairs (j, j + 4).
 // mf: the pair's field mask ((1 << BITS) - 1) * 0x10001 and ml (2 and 3
@@ -438,10 +448,28 @@ __device__ __forceinline__ uint32_t mma_funnel(const uint32_t* unit, int bit) {
   const int i0 = bit >> 5, i1 = i0 + 1 < BITS ? i0 + 1 : BITS - 1;
   return __builtin_amdgcn_alignbit(unit[i1], unit[i0], (uint32_t)(bit & 31));
 }
-template <int BITS>
+template <int BITS, typename XT>
 __device__ __forceinline__ u32x4_t mma_codes(const uint32_t* unit, int kb, uint32_t MB, uint32_t mf,
                                              uint32_t ml) {
-  if constexpr (BITS == 4) {
+  if constexpr (BITS == 8) {
+    // values j and j + 4 of the block are byte j of words 2 kb and 2 kb + 1
+    const uint32_t lo = unit[2 * kb], hi = unit[2 * kb + 1];
+    u32x4_t r;
+    if constexpr (Magic<8, XT>::dot2) {
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        r[j] = __builtin_amdgcn_perm(hi, lo, (uint32_t)j | 0x0C00u | ((uint32_t)(4 + j) << 16) | 0x0C000000u) | MB;
+    } else {
+      // bf16: 0..255 are exact in its 8 significant bits, so a code converts
+      // through fp32, whose upper half it is (no offset)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const float a = (float)((lo >> (8 * j)) & 0xFFu), b = (float)((hi >> (8 * j)) & 0xFFu);
+        r[j] = __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+      }
+    }
+    return r;
+  } else if constexpr (BITS == 4) {
     const uint32_t w = unit[kb];
     return u32x4_t{(w & mf) | MB, ((w >> 4) & mf) | MB, ((w >> 8) & mf) | MB, ((w >> 12) & mf) | MB};
   } else if constexpr (BITS <= 3) {
@@ -470,17 +498,21 @@ __device__ __forceinline__ u32x4_t mma_codes(const uint32_t* unit, int kb, uint3
 
 // Four waves per SIMD where that fits in 128 VGPRs without spills (2- and
 // 4-bit, 3-bit gate/up); the compiler's own choice elsewhere.
-template <int BITS, bool GATEUP>
-constexpr int kMmaWavesPerEu = (BITS == 2 || BITS == 4 || (BITS == 3 && GATEUP)) ? 4 : 1;
+template <int BITS, bool GATEUP, int TT>
+constexpr int kMmaWavesPerEu = TT == 2 ? 3 : (BITS == 2 || BITS == 4 || (BITS == 3 && GATEUP) || BITS == 8) ? 4 : 1;
 
 // GSH: log2(group size / 32), the launch's a.gsh (group sizes 32, 64, 128).
-template <int BITS, typename XT, typename ST, bool GATEUP, int GSH>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMmaWavesPerEu<BITS, GATEUP>)))
+// TT: 16-row activation tiles per pass (1 or 2).
+template <int BITS, typename XT, typename ST, bool GATEUP, int GSH, int TT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMmaWavesPerEu<BITS, GATEUP, TT>)))
 void gemv_mma_kernel(const GemvArgs a) {
-  __shared__ __align__(16) uint32_t wl[2][kMmaRows * kMmaU * BITS];  // [row][unit slot][BITS words]
-  __shared__ __align__(16) uint32_t sl[2][kMmaRows * kMmaU];      // [row][unit]: s | b << 16
-  __shared__ __align__(16) uint32_t xl[2][kMmaU * kMmaTok * 16];  // [unit][row][quad slot][4 words]
-  __shared__ float gl[32 * kMmaTok];                              // gate outputs of a pass
+  constexpr int kMmaTok = 16 * TT;  // activation rows per pass
+  constexpr int U = kMmaUnits<BITS>, NI = U / 4;  // staging items per thread
+  __shared__ __align__(16) uint32_t wl[2][kMmaRows * U * BITS];  // [row][unit slot][BITS words]
+  __shared__ __align__(16) uint32_t sl[2][kMmaRows * U];      // [row][group]: s | b << 16
+  __shared__ __align__(16) uint32_t xl[2][U * kMmaTok * 16];  // [unit][row][quad slot][4 words]
+  float* gl = reinterpret_cast<float*>(xl[0]);  // gate outputs of a pass (32 x kMmaTok), after its products
+  static_assert(32 * kMmaTok * 4 <= sizeof(xl[0]), "gate outputs fit a stage");
   const int slot = blockIdx.x / a.row_blocks, rb = blockIdx.x - slot * a.row_blocks;
   if ((uint32_t)slot >= a.used[0]) return;  // block-uniform, before any barrier
   const uint32_t e = __builtin_amdgcn_readfirstlane(a.used[1 + slot]);
@@ -488,11 +520,11 @@ void gemv_mma_kernel(const GemvArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int N = a.N, K = a.K, CU = K >> 5, groups = CU >> GSH, row_words = CU * BITS;
   constexpr int UPG = 1 << GSH;  // units per scale group
-  const int nchunks = (CU + kMmaU - 1) / kMmaU;
+  const int nchunks = (CU + U - 1) / U;
   constexpr int RPB = GATEUP ? 32 : 64;  // output rows per block
   const int r_begin = rb * RPB;
-  const ProjView P0 = proj_view<BITS, ST>(a.p0, e, N, row_words, groups);
-  const ProjView P1 = GATEUP ? proj_view<BITS, ST>(a.p1, e, N, row_words, groups) : P0;
+  // the projection whose rows this wave stages (and, for a pair, multiplies)
+  const ProjView PV = proj_view<BITS, ST>(GATEUP && wave >= 2 ? a.p1 : a.p0, e, N, row_words, groups);
   // activation rows through a buffer view (the host keeps x_rows K 16-bit
   // values below 2^31 bytes): the rows of a pass past its end read zero at a
   // dead offset instead of repeating its last row, and offsets stay 32-bit
@@ -500,22 +532,29 @@ void gemv_mma_kernel(const GemvArgs a) {
   // MAGIC + q is exact in the 16-bit type for q < 128 (bf16) / 1024 (f16)
   constexpr float MAGIC = Magic<BITS, XT>::value;
   constexpr uint32_t MB = Magic<BITS, XT>::bits;
-  static_assert(Magic<BITS, XT>::dot2, "magic-offset codes");
   const int r = lane & 15, kb = lane >> 4;
   // this lane's LDS weight row and output row
   const int lr = GATEUP ? (wave >> 1) * 32 + (wave & 1) * 16 + r : wave * 16 + r;
   const int orow = r_begin + (GATEUP ? (wave & 1) * 16 : wave * 16) + r;
 
-  // staging items of this thread, j < 2: codes and scales of LDS row
-  // (tid >> 3) + 32 j, unit slot tid & 7; activation quad q = tid + 256 j:
-  // unit q >> 6, row (q >> 2) & 15 (the same for both j), quad q & 3
-  const int s_lr0 = tid >> 3, s_us = tid & 7;
+  // staging items of this thread, j < NI: codes of LDS row slr_of(j), unit slot
+  // tid % U (waves 0-1 stage rows 0-31, the gate rows of a pair, waves 2-3 the
+  // rest); activation quad q = tid + 256 j: unit q >> 6, row (q >> 2) & 15 of
+  // each 16-row tile (the same for every j), quad q & 3
+  const int s_us = tid & (U - 1);
+  auto slr_of = [&](int j) -> int { return 32 * (tid >> 7) + ((tid & 127) / U) + 16 * j; };
   const int x_t = (tid >> 2) & 15, x_kb = tid & 3, x_us0 = wave;  // x_us0 scalar
+  // Groups of two or more units: the even unit of a pair loads the group's
+  // scale and bias for item 0's row, the odd one for item 1's: one load of each
+  // per thread and chunk instead of two. SI: scale items per thread.
+  constexpr bool kSbPairs = GSH >= 1 && NI == 2;
+  constexpr int SI = kSbPairs ? 1 : NI;
   struct Stage {
-    uint32_t w[2][BITS];
-    u32x4_t x[2];
-    uint32_t s[2], b[2];  // 16-bit scale and bias, merged only when stored (no early wait)
+    uint32_t w[NI][BITS];
+    u32x4_t x[TT][NI];
+    uint32_t s[SI], b[SI];  // 16-bit scale and bias, merged only when stored (no early wait)
   };
+  auto sb_row = [&](int i) -> int { return slr_of(kSbPairs ? (s_us & 1) : i); };
   auto gw_row = [&](int slr) -> uint32_t {
     const int g = GATEUP ? r_begin + (slr & 31) : r_begin + slr;
     return (uint32_t)min(g, N - 1);
@@ -527,55 +566,63 @@ void gemv_mma_kernel(const GemvArgs a) {
   auto load_w_stage = [&](int c, Stage& st) __attribute__((always_inline)) {
     const int cc = min(c, nchunks - 1);
     const uint32_t dead = c < nchunks ? 0u : 0x80000000u;  // block-uniform
+    const int uu = U * cc + s_us;
+    const uint32_t u = (uint32_t)min(uu, CU - 1);
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-      const int slr = s_lr0 + 32 * j;
-      const ProjView& pv = (GATEUP && j == 1) ? P1 : P0;
-      const uint32_t grow = gw_row(slr);
-      const int uu = kMmaU * cc + s_us;
-      const uint32_t u = (uint32_t)min(uu, CU - 1);
-      bload_unit<BITS>(pv.w, (grow * (uint32_t)row_words + u * (uint32_t)BITS) * 4u + dead, st.w[j]);
-      // units past K (the last chunk's tail) read a zero scale and bias, so
-      // their products with the clamped unit's codes and activations add
-      // zero (for finite activations; a non-finite one in a row's last unit
-      // makes its outputs non-finite either way)
-      const uint32_t sdead = uu < CU ? dead : 0x80000000u;
-      const uint32_t gi = (grow * (uint32_t)groups + (u >> GSH)) * (uint32_t)sizeof(ST) + sdead;
-      st.s[j] = (uint32_t)bload16(pv.s, gi);
-      st.b[j] = (uint32_t)bload16(pv.b, gi);
+    for (int j = 0; j < NI; j++)
+      bload_unit<BITS>(PV.w, (gw_row(slr_of(j)) * (uint32_t)row_words + u * (uint32_t)BITS) * 4u + dead, st.w[j]);
+    // units past K (the last chunk's tail) read a zero scale and bias, so
+    // their products with the clamped unit's codes and activations add
+    // zero (for finite activations; a non-finite one in a row's last unit
+    // makes its outputs non-finite either way)
+    const uint32_t sdead = uu < CU ? dead : 0x80000000u;
+#pragma unroll
+    for (int i = 0; i < SI; i++) {
+      const uint32_t gi = (gw_row(sb_row(i)) * (uint32_t)groups + (u >> GSH)) * (uint32_t)sizeof(ST) + sdead;
+      st.s[i] = (uint32_t)bload16(PV.s, gi);
+      st.b[i] = (uint32_t)bload16(PV.b, gi);
     }
   };
-  auto load_x_stage = [&](int c, uint32_t xbase, Stage& st) __attribute__((always_inline)) {
+  auto load_x_stage = [&](int c, const uint32_t (&xbase)[TT], Stage& st) __attribute__((always_inline)) {
     const int cc = min(c, nchunks - 1);
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-      const int ux = min(kMmaU * cc + x_us0 + 4 * j, CU - 1);
-      st.x[j] = bload128(xr, xbase + (uint32_t)ux * 64u + (uint32_t)x_kb * 16u);
+    for (int j = 0; j < NI; j++) {
+      const int ux = min(U * cc + x_us0 + 4 * j, CU - 1);
+#pragma unroll
+      for (int tt = 0; tt < TT; tt++)
+        st.x[tt][j] = bload128(xr, xbase[tt] + (uint32_t)ux * 64u + (uint32_t)x_kb * 16u);
     }
   };
-  auto load_stage = [&](int c, uint32_t xbase, Stage& st) __attribute__((always_inline)) {
+  auto load_stage = [&](int c, const uint32_t (&xbase)[TT], Stage& st) __attribute__((always_inline)) {
     load_w_stage(c, st);
     load_x_stage(c, xbase, st);
   };
   auto store_stage = [&](const Stage& st, int buf) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-      const int slr = s_lr0 + 32 * j;
-      uint32_t* wd = &wl[buf][(slr * kMmaU + ((s_us + slr) & 7)) * BITS];
-      if constexpr (BITS == 4) {
-        *reinterpret_cast<u32x4_t*>(wd) = u32x4_t{st.w[j][0], st.w[j][1], st.w[j][2], st.w[j][3]};
+    for (int j = 0; j < NI; j++) {
+      const int slr = slr_of(j);
+      uint32_t* wd = &wl[buf][(slr * U + ((s_us + slr) & (U - 1))) * BITS];
+      if constexpr (BITS % 4 == 0) {
+#pragma unroll
+        for (int q = 0; q < BITS; q += 4)
+          *reinterpret_cast<u32x4_t*>(wd + q) = u32x4_t{st.w[j][q], st.w[j][q + 1], st.w[j][q + 2], st.w[j][q + 3]};
       } else {
 #pragma unroll
         for (int q = 0; q < BITS; q++) wd[q] = st.w[j][q];
       }
-      sl[buf][slr * kMmaU + s_us] = st.s[j] | (st.b[j] << 16);
       // natural values x0..x7 -> pairs (x0, x4), (x1, x5), (x2, x6), (x3, x7)
-      const u32x4_t n = st.x[j];
-      const u32x4_t pw = {(n[0] & 0xFFFFu) | (n[2] << 16), (n[0] >> 16) | (n[2] & 0xFFFF0000u),
-                          (n[1] & 0xFFFFu) | (n[3] << 16), (n[1] >> 16) | (n[3] & 0xFFFF0000u)};
-      const int us = x_us0 + 4 * j;
-      *reinterpret_cast<u32x4_t*>(&xl[buf][((us * kMmaTok + x_t) * 4 + (x_kb ^ ((x_t >> 2) & 3))) * 4]) = pw;
+#pragma unroll
+      for (int tt = 0; tt < TT; tt++) {
+        const u32x4_t n = st.x[tt][j];
+        const u32x4_t pw = {(n[0] & 0xFFFFu) | (n[2] << 16), (n[0] >> 16) | (n[2] & 0xFFFF0000u),
+                            (n[1] & 0xFFFFu) | (n[3] << 16), (n[1] >> 16) | (n[3] & 0xFFFF0000u)};
+        const int us = x_us0 + 4 * j;
+        *reinterpret_cast<u32x4_t*>(
+            &xl[buf][((us * kMmaTok + 16 * tt + x_t) * 4 + (x_kb ^ ((x_t >> 2) & 3))) * 4]) = pw;
+      }
     }
+#pragma unroll
+    for (int i = 0; i < SI; i++) sl[buf][sb_row(i) * U + (s_us >> GSH)] = st.s[i] | (st.b[i] << 16);
   };
   const u32x4_t ones = {Mma16<XT>::ones, Mma16<XT>::ones, Mma16<XT>::ones, Mma16<XT>::ones};
   // opaque copies of the unpack's constants (see mma_codes)
@@ -583,7 +630,7 @@ void gemv_mma_kernel(const GemvArgs a) {
   asm("s_mov_b32 %0, %1" : "=s"(mf) : "i"(((1u << BITS) - 1u) * 0x10001u));
   asm("s_mov_b32 %0, %1" : "=s"(ml) : "i"((1u << (4 * (BITS < 4 ? BITS : 4))) - 1u));
   asm("v_mov_b32 %0, %1" : "=v"(mbv) : "i"(MB));
-  f32x4_t acc;
+  f32x4_t acc[TT];
   // Every chunk runs the same straight-line code: K is a multiple of the
   // group size, so groups never straddle the end of K, and the units past it
   // carry zero scales and biases. A group's first unit starts P and Q from a
@@ -591,22 +638,28 @@ void gemv_mma_kernel(const GemvArgs a) {
   // scale and bias; with the group size a runtime value the compiler kept
   // both per unit behind branches, with eight register clears per group.
   auto compute = [&](int buf) __attribute__((always_inline)) {
-    f32x4_t P = {}, Q = {};
+    f32x4_t P[TT] = {}, Q[TT] = {};
 #pragma unroll
-    for (int us = 0; us < kMmaU; us++) {
-      const u32x4_t bop = mma_codes<BITS>(&wl[buf][(lr * kMmaU + ((us + lr) & 7)) * BITS], kb, mbv, mf, ml);
-      const u32x4_t aop =
-          *reinterpret_cast<const u32x4_t*>(&xl[buf][((us * kMmaTok + r) * 4 + (kb ^ ((r >> 2) & 3))) * 4]);
-      P = Mma16<XT>::mma(aop, bop, us % UPG == 0 ? f32x4_t{} : P);
-      Q = Mma16<XT>::mma(aop, ones, us % UPG == 0 ? f32x4_t{} : Q);
+    for (int us = 0; us < U; us++) {
+      const u32x4_t bop = mma_codes<BITS, XT>(&wl[buf][(lr * U + ((us + lr) & (U - 1))) * BITS], kb, mbv, mf, ml);
+#pragma unroll
+      for (int tt = 0; tt < TT; tt++) {
+        const u32x4_t aop = *reinterpret_cast<const u32x4_t*>(
+            &xl[buf][((us * kMmaTok + 16 * tt + r) * 4 + (kb ^ ((r >> 2) & 3))) * 4]);
+        P[tt] = Mma16<XT>::mma(aop, bop, us % UPG == 0 ? f32x4_t{} : P[tt]);
+        Q[tt] = Mma16<XT>::mma(aop, ones, us % UPG == 0 ? f32x4_t{} : Q[tt]);
+      }
       if ((us + 1) % UPG == 0) {
-        const uint32_t sb = sl[buf][lr * kMmaU + us];
+        const uint32_t sb = sl[buf][lr * U + (us >> GSH)];
         const float sc = to_f<ST>(__builtin_bit_cast(ST, (uint16_t)(sb & 0xFFFFu)));
         const float bi = to_f<ST>(__builtin_bit_cast(ST, (uint16_t)(sb >> 16))) - MAGIC * sc;
         // two chained fmas per output (the sum s P + bi Q as written cost a
         // multiply, an fma and an add)
 #pragma unroll
-        for (int i = 0; i < 4; i++) acc[i] = __builtin_fmaf(bi, Q[i], __builtin_fmaf(sc, P[i], acc[i]));
+        for (int tt = 0; tt < TT; tt++)
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            acc[tt][i] = __builtin_fmaf(bi, Q[tt][i], __builtin_fmaf(sc, P[tt][i], acc[tt][i]));
       }
     }
   };
@@ -623,16 +676,22 @@ void gemv_mma_kernel(const GemvArgs a) {
   const uint32_t pend = __builtin_amdgcn_readfirstlane(a.offsets[e + 1]);
   for (uint32_t pc = pbeg; pc < pend; pc += kMmaTok) {
     const int nt = min((int)(pend - pc), kMmaTok);
-    const uint32_t p = pc + (uint32_t)min(x_t, nt - 1);
-    const uint32_t xrow = a.perm ? a.perm[p] / (uint32_t)a.topk : p;
-    const uint32_t xbase = x_t < nt ? xrow * (uint32_t)K * (uint32_t)sizeof(XT) : 0x80000000u;
+    uint32_t xbase[TT];
+#pragma unroll
+    for (int tt = 0; tt < TT; tt++) {
+      const int t = 16 * tt + x_t;
+      const uint32_t p = pc + (uint32_t)min(t, nt - 1);
+      const uint32_t xrow = a.perm ? a.perm[p] / (uint32_t)a.topk : p;
+      xbase[tt] = t < nt ? xrow * (uint32_t)K * (uint32_t)sizeof(XT) : 0x80000000u;
+    }
     load_x_stage(0, xbase, s0);
     load_x_stage(1, xbase, s1);
     lds_barrier();  // the last pass's LDS reads (and gl) are done; loads stay in flight
     store_stage(s0, 0);
     load_stage(2, xbase, s0);
     lds_barrier();
-    acc = f32x4_t{};
+#pragma unroll
+    for (int tt = 0; tt < TT; tt++) acc[tt] = f32x4_t{};
     // No break in this loop: with one, the compiler's wait counts at the loop
     // head took the break path's state (chunk c + 3's loads youngest) and the
     // stores of chunk c + 1 waited for chunk c + 2's loads as well. An odd
@@ -649,25 +708,25 @@ void gemv_mma_kernel(const GemvArgs a) {
       load_stage(c + 4, xbase, s0);
       lds_barrier();
     }
-    // lane (r, kb): output column orow, activation rows 4 kb + i of the pass
+    // lane (r, kb): output column orow, activation rows 16 tt + 4 kb + i of the pass
     const size_t ob_i = (size_t)e * N + (size_t)min(orow, N - 1);
     if constexpr (GATEUP) {
       if (wave < 2) {
         const float ob = a.p0.ob ? to_f<XT>(reinterpret_cast<const XT*>(a.p0.ob)[ob_i]) : 0.f;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          float g = round_to<XT>(acc[i]);
+        for (int i = 0; i < 4 * TT; i++) {
+          float g = round_to<XT>(acc[i >> 2][i & 3]);
           if (a.p0.ob) g = round_to<XT>(g + ob);
-          gl[((wave & 1) * 16 + r) * kMmaTok + 4 * kb + i] = g;
+          gl[((wave & 1) * 16 + r) * kMmaTok + 16 * (i >> 2) + 4 * kb + (i & 3)] = g;
         }
       }
       __syncthreads();
       if (wave >= 2) {
         const float ob = a.p1.ob ? to_f<XT>(reinterpret_cast<const XT*>(a.p1.ob)[ob_i]) : 0.f;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const int t = 4 * kb + i;
-          float u = round_to<XT>(acc[i]);
+        for (int i = 0; i < 4 * TT; i++) {
+          const int t = 16 * (i >> 2) + 4 * kb + (i & 3);
+          float u = round_to<XT>(acc[i >> 2][i & 3]);
           if (a.p1.ob) u = round_to<XT>(u + ob);
           const float g = gl[((wave & 1) * 16 + r) * kMmaTok + t];
           if (t < nt && orow < N)
@@ -677,9 +736,9 @@ void gemv_mma_kernel(const GemvArgs a) {
     } else {
       const float ob = a.p0.ob ? to_f<XT>(reinterpret_cast<const XT*>(a.p0.ob)[ob_i]) : 0.f;
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int t = 4 * kb + i;
-        float g = round_to<XT>(acc[i]);
+      for (int i = 0; i < 4 * TT; i++) {
+        const int t = 16 * (i >> 2) + 4 * kb + (i & 3);
+        float g = round_to<XT>(acc[i >> 2][i & 3]);
         if (a.p0.ob) g = round_to<XT>(g + ob);
         // single projection: only ReLU^2 acts on it (no gate)
         const float v = a.act == ACT_RELU2 ? apply_act<XT>(0.f, g, ACT_RELU2, 0.f, 0.f) : g;
@@ -693,15 +752,23 @@ void gemv_mma_kernel(const GemvArgs a) {
   }
 }
 
-template <typename XT, typename ST, int GSH>
-static hipError_t launch_mma_g(bool gateup, const GemvArgs& a, int grid, hipStream_t st, KEvents ev) {
+template <typename XT, typename ST, int GSH, int TT>
+static hipError_t launch_mma_t(bool gateup, const GemvArgs& a, int grid, hipStream_t st, KEvents ev) {
   if (gateup)
-    hipExtLaunchKernelGGL((gemv_mma_kernel<MOE_BITS, XT, ST, true, GSH>), dim3(grid), dim3(256), 0, st,
+    hipExtLaunchKernelGGL((gemv_mma_kernel<MOE_BITS, XT, ST, true, GSH, TT>), dim3(grid), dim3(256), 0, st,
                           ev.start, ev.stop, 0, a);
   else
-    hipExtLaunchKernelGGL((gemv_mma_kernel<MOE_BITS, XT, ST, false, GSH>), dim3(grid), dim3(256), 0, st,
+    hipExtLaunchKernelGGL((gemv_mma_kernel<MOE_BITS, XT, ST, false, GSH, TT>), dim3(grid), dim3(256), 0, st,
                           ev.start, ev.stop, 0, a);
   return hipGetLastError();
+}
+// a.tok_chunk: activation rows per pass, 16 or 32 (32 built for 4 and 8 bits,
+// the widths of nearly every checkpoint; the others take 16)
+template <typename XT, typename ST, int GSH>
+static hipError_t launch_mma_g(bool gateup, const GemvArgs& a, int grid, hipStream_t st, KEvents ev) {
+  if constexpr (MOE_BITS == 4 || MOE_BITS == 8)
+    if (a.tok_chunk > 16) return launch_mma_t<XT, ST, GSH, 2>(gateup, a, grid, st, ev);
+  return launch_mma_t<XT, ST, GSH, 1>(gateup, a, grid, st, ev);
 }
 
 hipError_t MOE_CAT(launch_mma_b, MOE_BITS)(int xdt, int sbdt, bool gateup, const GemvArgs& a,
@@ -720,7 +787,6 @@ hipError_t MOE_CAT(launch_mma_b, MOE_BITS)(int xdt, int sbdt, bool gateup, const
 #undef MOE_MMA
   return hipErrorInvalidValue;
 }
-#endif  // MOE_BITS <= 6
 
 // ---------------------------------------------------------------------------
 // one activation row per expert (decode T = 1): activations live in registers

@@ -334,6 +334,48 @@ def test_expert_matmul_tile_edges(bits, dt, sb, gs, K, counts, N):
         check_close(got, ref, dt, f"tile edges bits={bits} gs={gs} K={K} rows={counts} N={N}")
 
 
+@pytest.mark.parametrize("bits,dt,sb,gs,K", [
+    (8, BF16, BF16, 64, 320),   # 8-bit codes as plain bf16 integers
+    (8, BF16, F16, 32, 96),     # fewer units than a chunk
+    (8, F16, F16, 128, 640),    # 1024 + code in f16
+    (8, F16, BF16, 32, 1056),
+    (4, BF16, BF16, 64, 448),   # a last chunk of 6 units
+    (4, F16, F16, 128, 384),
+    (3, BF16, BF16, 64, 576),
+    (6, BF16, F16, 32, 288),
+])
+@pytest.mark.parametrize("counts", [(2, 5, 1), (16, 1, 17), (17, 33, 16), (0, 32, 31)])
+@pytest.mark.parametrize("N", [24, 65])
+def test_expert_matmul_mma_gemv(bits, dt, sb, gs, K, counts, N):
+    """The batched matrix-core GEMV at one row, a full and an overfull pass of
+    16 and 32 rows, partial weight-row blocks and partial K chunks. Tolerance:
+    the layer bar (no operand is rounded: the bar allows the output's own
+    rounding)."""
+    from moe_spec import gen_qproj
+    rng = np.random.default_rng(bits * 1000 + K + N + sum(counts))
+    E, M = len(counts), int(sum(counts))
+    f = 15.0 / (2 ** bits - 1)
+    p = gen_qproj(rng, E, N, K, bits, gs, sb, s_range=(0.005 * f, 0.02 * f))
+    experts = np.repeat(np.arange(E), counts).astype(np.uint32)
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32)
+    a = store(rng.normal(0, 1, (M, K)), dt)
+    lib = _lib.load()
+    q = _lib.QProj(0, 0, 0, None, bits, gs, sb, N, K, E)
+    wt, st, bt = to_torch(p.weight.view(np.int32)), to_torch(p.scales), to_torch(p.biases)
+    q.weight, q.scales, q.biases = wt.data_ptr(), st.data_ptr(), bt.data_ptr()
+    at = to_torch(a)
+    out = torch.empty(M, N, dtype=at.dtype, device="cuda")
+    wsb = lib.moe_expert_matmul_workspace_bytes(C.byref(q), dt, M)
+    ws = torch.empty(wsb, dtype=torch.uint8, device="cuda")
+    offt = to_torch(offsets.view(np.int32))
+    for _ in range(2):
+        check(lib.moe_expert_matmul(C.byref(q), _p(at), dt, None, 1, M, _p(offt), _p(out), _p(ws), wsb,
+                                    _stream()))
+        torch.cuda.synchronize()
+        ref = orc.round_dt(orc.qgemm_rows(p, load(a, dt), experts), dt)
+        check_close(to_numpy_f32(out), ref, dt, f"mma gemv bits={bits} gs={gs} K={K} rows={counts} N={N}")
+
+
 def test_gemm_operand_range_bf16():
     """The matrix-core path feeds a bf16 input to the matrix cores as f16
     values x 2^-8, converted to nearest: a row element at 2^25 (beyond
