@@ -23,6 +23,10 @@ constexpr int kPlanThreads = 256;
 constexpr int kPlanMaxE = 1024;
 constexpr int kChunk = 1024;             // entries per chunk in the multi-block plan
 constexpr int kSingleBlockMax = 4096;    // M at or below which one workgroup plans
+// Entries for which a block per expert plans (plan_experts_kernel): up to the
+// ids 1024 threads hold in 32 registers each; from 512 entries one workgroup
+// (4.8 us there) takes longer than the 5 us it takes at any count up to 4096.
+constexpr int kPlanExpertsMin = 512, kPlanExpertsMax = 32768;
 
 // Exclusive scan of cnt[0..E) over NT threads (4 experts per thread).
 // Writes offsets[0..E], counts, the used list, and base[e] = offsets[e].
@@ -255,6 +259,121 @@ hipError_t launch_route_plan(const void* logits, int dt, int T, int E, int k, co
   return hipErrorInvalidValue;
 }
 
+// The whole plan in one launch, a block per expert: every block reads all M ids
+// (held in registers, 4 QUADS per thread; 1024 threads, each wave a contiguous
+// share so that wave and lane order are token order), counts those below its
+// expert (its offset) and its own, and writes its own entries in order. The
+// E M id reads come from L2 (128 experts, 32768 ids: 16.8 MB) and cost less than
+// the launches, the one-block scan and the waves' turns at the cursors that one
+// workgroup or three passes over chunks take (us: 1998 ids 11.8 -> 5.0, 4000
+// ids with the GEMM's row tiles 16.6 + 5.6 -> 5.5, 16384 ids on 256 experts
+// 5.3 + 5.5 + 9.8 -> 6.3, 32768 on 128 experts 4.9 + 4.9 + 10.6 -> 9.0).
+// items (nullable): also the GEMM's row tiles. Expert e's tiles start at slot
+// offset / kGemmTileRows + e, which leaves room for every tile before them
+// (ceil(c / R) <= floor((o + c) / R) - floor(o / R) + 1); a slot without a tile
+// holds no rows (kGemmNoTile).
+// used (nullable): the used list, which needs the experts below e that occur:
+// a bitmap of them.
+template <int QUADS>
+__global__ __launch_bounds__(1024) void plan_experts_kernel(
+    const uint32_t* __restrict__ idx, int M, int E, uint32_t* __restrict__ counts,
+    uint32_t* __restrict__ offsets, uint32_t* __restrict__ perm, uint32_t* __restrict__ inv,
+    uint32_t* __restrict__ used, uint32_t* __restrict__ items) {
+  __shared__ uint32_t wlt[16], weq[16];
+  __shared__ uint32_t seen[kPlanMaxE / 32];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t e = blockIdx.x;
+  const rsrc_t iv = make_rsrc(idx, (uint32_t)M * 4u);
+  // quad q of this lane: entries 4 ((wave QUADS + q) 64 + lane) + c
+  u32x4_t id[QUADS];
+#pragma unroll
+  for (int q = 0; q < QUADS; q++) id[q] = bload128(iv, (uint32_t)((wave * QUADS + q) * 64 + lane) * 16u);
+  if (used && tid < kPlanMaxE / 32) seen[tid] = 0;
+  uint32_t lt = 0, eq = 0;
+#pragma unroll
+  for (int q = 0; q < QUADS; q++)
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      const int m = 4 * ((wave * QUADS + q) * 64 + lane) + c;
+      if (m >= M) id[q][c] = 0xFFFFFFFFu;  // past the end the view reads zeros
+      lt += id[q][c] < e ? 1u : 0u;
+      eq += id[q][c] == e ? 1u : 0u;
+    }
+  const uint32_t slt = wave_scan_u32(lt), seq = wave_scan_u32(eq);
+  if (lane == 63) {
+    wlt[wave] = slt;
+    weq[wave] = seq;
+  }
+  __syncthreads();
+  uint32_t off = 0, n = 0, at = 0;
+#pragma unroll
+  for (int w = 0; w < 16; w++) {
+    const uint32_t a = wlt[w], b = weq[w];
+    off += a;
+    n += b;
+    at += w < wave ? b : 0u;
+  }
+  if (used) {
+#pragma unroll
+    for (int q = 0; q < QUADS; q++)
+#pragma unroll
+      for (int c = 0; c < 4; c++)
+        if (id[q][c] < e) atomicOr(&seen[id[q][c] >> 5], 1u << (id[q][c] & 31u));
+  }
+  // this wave's entries of the expert, in order: quad by quad, lane by lane
+  uint32_t run = off + at;
+#pragma unroll
+  for (int q = 0; q < QUADS; q++) {
+    uint64_t b[4];
+    uint32_t before = 0, all = 0;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      b[c] = __ballot(id[q][c] == e);
+      before += __builtin_amdgcn_mbcnt_hi((uint32_t)(b[c] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b[c], 0u));
+      all += (uint32_t)__popcll(b[c]);
+    }
+    uint32_t p = run + before;
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      if (id[q][c] == e) {
+        const uint32_t m = (uint32_t)(4 * ((wave * QUADS + q) * 64 + lane) + c);
+        perm[p] = m;
+        inv[m] = p;
+        p++;
+      }
+    }
+    run += all;
+  }
+  if (tid == 0) {
+    counts[e] = n;
+    offsets[e] = off;
+    if (e == (uint32_t)E - 1u) offsets[E] = off + n;
+  }
+  if (items) {
+    constexpr uint32_t R = kGemmTileRows;
+    const uint32_t first = off / R + e, end = (e == (uint32_t)E - 1u) ? (uint32_t)M / R + (uint32_t)E : (off + n) / R + e + 1u;
+    for (uint32_t t = (uint32_t)tid; t < end - first; t += 1024u) {
+      const uint32_t r = t * R;
+      const bool live = r < n;
+      items[4 + 2 * (first + t)] = live ? e : kGemmNoTile;
+      items[5 + 2 * (first + t)] = live ? (off + r) | ((min(n - r, R) - 1u) << 25) : 0u;
+    }
+    if (e == (uint32_t)E - 1u && tid == 0) items[0] = end;
+  }
+  if (used) {
+    __syncthreads();
+    if (wave == 0) {
+      const uint32_t w = lane < kPlanMaxE / 32 ? (uint32_t)__popc(seen[lane]) : 0u;
+      const uint32_t rank = (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_u32(w), 63);
+      if (lane == 0) {
+        if (n) used[1 + rank] = e;
+        if (e == (uint32_t)E - 1u) used[0] = rank + (n ? 1u : 0u);
+      }
+    }
+  }
+}
+
 // Multi-block pass 1: per-chunk histograms, hist[c * E + e].
 __global__ __launch_bounds__(kPlanThreads) void plan_hist_kernel(const uint32_t* __restrict__ idx,
                                                                  int M, int E,
@@ -433,6 +552,18 @@ hipError_t launch_dispatch_plan(const uint32_t* idx, int T, int k, int E, uint32
   if (items_done) *items_done = false;
   const int M = T * k;
   if (E > kPlanMaxE) return hipErrorInvalidValue;
+  if (M > kPlanExpertsMin && M <= kPlanExpertsMax) {
+#define MOE_PE(QUADS)                                                                              \
+  hipLaunchKernelGGL((plan_experts_kernel<QUADS>), dim3(E), dim3(1024), 0, st, idx, M, E, counts,   \
+                     offsets, perm, inv_perm, items ? nullptr : used, items)
+    if (M <= 4096) MOE_PE(1);
+    else if (M <= 8192) MOE_PE(2);
+    else if (M <= 16384) MOE_PE(4);
+    else MOE_PE(8);
+#undef MOE_PE
+    if (items_done) *items_done = items != nullptr;
+    return hipGetLastError();
+  }
   if (M <= kSingleBlockMax) {
     hipLaunchKernelGGL(plan_single_kernel, dim3(1), dim3(kPlanThreads), 0, st, idx, M, E, counts,
                        offsets, perm, inv_perm, used);

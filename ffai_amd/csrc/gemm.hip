@@ -636,6 +636,7 @@ __global__ __launch_bounds__(256, 3) void gemm_grouped_kernel(const GemmArgs a) 
   if (wi >= n) return;
   const uint32_t t = wi / nb;
   const uint32_t e = __builtin_amdgcn_readfirstlane(a.items[4 + 2 * t]);
+  if (e == kGemmNoTile) return;
   const uint32_t x1 = __builtin_amdgcn_readfirstlane(a.items[5 + 2 * t]);
   const uint32_t m0 = x1 & 0x1FFFFFFu, rows = (x1 >> 25) + 1u;
   const int bn = (int)(wi - t * nb);

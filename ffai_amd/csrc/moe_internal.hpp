@@ -270,9 +270,11 @@ inline int gemm_col_blocks(int N, bool gateup) {
 // Upper bound on the row tiles of a plan of M rows over E experts.
 inline long gemm_max_tiles(int M, int E) { return M / kGemmTileRows + (long)E; }
 inline size_t gemm_items_bytes(int M, int E) { return (size_t)(4 + 2 * gemm_max_tiles(M, E)) * 4; }
-// The row tiles of a plan: items[0] = count (items[1..3] unused), then 8
-// bytes per tile: expert, first sorted position | (rows - 1) << 25 (at most
-// 2^25 positions): experts ascending, an expert's tiles in order.
+// The row tiles of a plan: items[0] = slots (items[1..3] unused), then 8
+// bytes per slot: expert (kGemmNoTile: an empty slot), first sorted position |
+// (rows - 1) << 25 (at most 2^25 positions): experts ascending, an expert's
+// tiles in order.
+constexpr uint32_t kGemmNoTile = 0xFFFFFFFFu;
 hipError_t launch_gemm_items(const uint32_t* offsets, int E, uint32_t* items, hipStream_t st);
 // grid: 8 * ceil(gemm_max_tiles * col_blocks / 8) blocks (the (tile, column
 // block) pairs are split evenly over the XCDs at run time; blocks without one

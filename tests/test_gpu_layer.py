@@ -136,6 +136,8 @@ def test_router_logits_within_one_ulp(dt, wdt, E, H, T):
     (64, 128, 2048, 64, BF16, False),  # many tokens: the matrix-core kernel
     (96, 64, 768, 128, F16, True),
     (40, 40, 512, 64, BF16, True),     # many tokens, E % 32 != 0: the row kernel
+    (2016, 128, 128, 64, BF16, False), # 252 tiles: 16 waves per tile, 2 chunks
+    (2048, 128, 192, 32, F16, True),   # 256 tiles: 4 waves per tile
 ])
 def test_router_logits_q(bits, T, E, H, gs, dt, bias):
     """moe_router_logits_q (an mlx QuantizedLinear router) against the oracle's
@@ -184,6 +186,37 @@ def test_layer_quantised_shared_gate(mixed, T):
     """A 4-bit router and a 4-bit shared_expert_gate (Qwen3xText.swift:660-661,
     947-951) on the mixed-bit layer."""
     run_layer(with_quantised_router(mixed, bits=4, shared_gate_bits=4), T, seed=T + 1)
+
+
+@pytest.mark.parametrize("M,E", [(512, 16), (513, 5), (4096, 1), (4097, 300), (8193, 64), (16385, 1024),
+                                 (32768, 7), (32769, 40)])
+def test_dispatch_plan_edges(M, E):
+    """Entry counts around the plan's launch shapes (one workgroup, a block
+    per expert at 1, 2, 4 and 8 entries per thread and lane quad, the
+    chunked passes past 32768), k = 1, unused experts, and dropped ids."""
+    rng = np.random.default_rng(M + E)
+    idx = rng.integers(0, E, M).astype(np.uint32)
+    if E > 4:
+        idx[idx == 3] = 2                # an expert without entries
+    idx[rng.random(M) < 0.02] = E + 5    # out of range: dropped
+    lib = _lib.load()
+    out = {n: torch.full((sz,), -1, dtype=torch.int32, device="cuda")
+           for n, sz in (("counts", E), ("offsets", E + 1), ("perm", M), ("inv", M))}
+    wsb = lib.moe_dispatch_workspace_bytes(M, 1, E)
+    ws = torch.empty(max(wsb, 1), dtype=torch.uint8, device="cuda")
+    idxt = to_torch(idx.view(np.int32))
+    check(lib.moe_dispatch_plan(_p(idxt), M, 1, E, _p(out["counts"]), _p(out["offsets"]), _p(out["perm"]),
+                                _p(out["inv"]), _p(ws), wsb, _stream()))
+    torch.cuda.synchronize()
+    kept = np.nonzero(idx < E)[0]
+    order = kept[np.argsort(idx[kept], kind="stable")]
+    counts = np.bincount(idx[kept], minlength=E)
+    assert np.array_equal(_u32(out["counts"]), counts)
+    assert np.array_equal(_u32(out["offsets"]), np.concatenate([[0], np.cumsum(counts)]))
+    assert np.array_equal(_u32(out["perm"])[:len(order)], order)
+    inv = _u32(out["inv"])
+    assert np.array_equal(inv[order], np.arange(len(order)))
+    assert np.all(inv[idx >= E] == 0xFFFFFFFF)  # left unwritten
 
 
 @pytest.mark.parametrize("T,k,E", [(1, 8, 128), (1, 4, 32), (16, 2, 8), (64, 8, 128), (512, 8, 128),
