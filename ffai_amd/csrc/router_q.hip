@@ -16,7 +16,7 @@
 //    lane l takes units l + 64 j of the expert's row (v_dot2 over code pairs,
 //    as the decode GEMVs do);
 //  - router_qgemm_kernel, many tokens: a 32-token x 32-expert tile per block
-//    on v_mfma_f32_32x32x16, the four waves splitting the hidden dimension in
+//    on v_mfma_f32_32x32x16, the four or 16 waves splitting the hidden dimension in
 //    64-value chunks; per 32 values one MFMA pair gives sum((MAGIC + q) x) and
 //    one against all-ones gives sum(x), so the scale and bias of each unit
 //    apply in fp32 to a fresh partial product.
@@ -74,7 +74,11 @@ __global__ __launch_bounds__(256) void router_qrow_kernel(const XT* __restrict__
 
 // ------------------------------------------------------------ many tokens --
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
-constexpr int kRqWaves = 4;
+// Tiles of a launch below which a tile's hidden dimension goes over 16 waves
+// instead of 4: with few blocks the launch lasts as long as one wave's chain of
+// chunks (48 tokens, 64 experts of hidden 1024 at 8 bits, 16 chunks: 9.9 ->
+// 7.5 us).
+constexpr int kRqFewTiles = 256;
 
 template <typename XT> struct RqMfma;
 template <> struct RqMfma<bf16_t> {
@@ -137,13 +141,13 @@ __device__ __forceinline__ u32x4_t code_frag(const uint32_t (&w)[BITS], int v0) 
   return r;
 }
 
-template <int BITS, typename XT, typename ST>
-__global__ __launch_bounds__(64 * kRqWaves) void router_qgemm_kernel(const XT* __restrict__ x,
+template <int BITS, typename XT, typename ST, int NW>
+__global__ __launch_bounds__(64 * NW) void router_qgemm_kernel(const XT* __restrict__ x,
                                                                     const GemvProj W,
                                                                     const XT* __restrict__ bias,
                                                                     XT* __restrict__ logits, int T,
                                                                     int H, int E, int gsh) {
-  __shared__ float part[kRqWaves][32 * 33];
+  __shared__ float part[NW][32 * 33];
   constexpr float MAGIC = Magic<BITS, XT>::value;
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -160,7 +164,7 @@ __global__ __launch_bounds__(64 * kRqWaves) void router_qgemm_kernel(const XT* _
   const uint32_t wo = ex * (uint32_t)row_words * 4u;
   const uint32_t so = ex * (uint32_t)groups;
   const int G = H >> 6;
-  const int ng = (G - wv + kRqWaves - 1) / kRqWaves;  // chunks wv + 4 i, i < ng
+  const int ng = (G - wv + NW - 1) / NW;  // chunks wv + 4 i, i < ng
 
   struct Set {
     u32x4_t a[4];
@@ -168,7 +172,7 @@ __global__ __launch_bounds__(64 * kRqWaves) void router_qgemm_kernel(const XT* _
     ST s[2], b[2];
   };
   auto load = [&](int i, Set& st) __attribute__((always_inline)) {
-    const int c = min(wv + kRqWaves * i, G - 1);  // clamped: in bounds, never multiplied
+    const int c = min(wv + NW * i, G - 1);  // clamped: in bounds, never multiplied
     const uint32_t kb = (uint32_t)c * 128u;
 #pragma unroll
     for (int q = 0; q < 4; q++) st.a[q] = bload128(xr, xo + kb + 32u * (uint32_t)q);
@@ -216,12 +220,12 @@ __global__ __launch_bounds__(64 * kRqWaves) void router_qgemm_kernel(const XT* _
   for (int r = 0; r < 16; r++) part[wv][(8 * (r >> 2) + 4 * h + (r & 3)) * 33 + col] = acc[r];
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < 1024 / (64 * kRqWaves); j++) {
-    const int o = threadIdx.x + 64 * kRqWaves * j;
+  for (int j = 0; j < 1024 / (64 * NW); j++) {
+    const int o = threadIdx.x + 64 * NW * j;
     const int r = o >> 5, c = o & 31;
     float v = part[0][r * 33 + c];
 #pragma unroll
-    for (int w = 1; w < kRqWaves; w++) v += part[w][r * 33 + c];
+    for (int w = 1; w < NW; w++) v += part[w][r * 33 + c];
     if (t0 + r < T && e0 + c < E) {
       float l = round_to<XT>(v);
       if (bias) l = round_to<XT>(l + to_f<XT>(bias[e0 + c]));
@@ -237,9 +241,13 @@ static hipError_t launch_rq_t(const void* x, int T, int H, const GemvProj& W, in
   // the matrix-core kernel views x as one buffer with 32-bit offsets: beyond
   // 4 GiB of input rows the per-row kernel (64-bit row addresses) runs
   if (T >= 32 && H % 64 == 0 && (size_t)T * H * sizeof(XT) < (1ull << 32)) {
-    hipLaunchKernelGGL((router_qgemm_kernel<BITS, XT, ST>), dim3((T + 31) / 32, (E + 31) / 32),
-                       dim3(64 * kRqWaves), 0, st, (const XT*)x, W, (const XT*)bias, (XT*)logits,
-                       T, H, E, gsh);
+    const dim3 grid((T + 31) / 32, (E + 31) / 32);
+#define MOE_RQG(NW)                                                                             \
+  hipLaunchKernelGGL((router_qgemm_kernel<BITS, XT, ST, NW>), grid, dim3(64 * NW), 0, st,       \
+                     (const XT*)x, W, (const XT*)bias, (XT*)logits, T, H, E, gsh)
+    if ((int)(grid.x * grid.y) < kRqFewTiles) MOE_RQG(16);
+    else MOE_RQG(4);
+#undef MOE_RQG
     return hipGetLastError();
   }
   const int tchunks = (T + 7) / 8;
