@@ -473,6 +473,17 @@ struct Workspace {
   size_t total;
 };
 
+// Bytes a workspace holds for the GEMM's list over N outputs: 16 per 256-row
+// tile and 128 (gate/up) or 256 columns, more than two such regions' tile list
+// needs (8 bytes per 96-row tile: M / 12 + 8 E against M / 8 + 32 E at one
+// column block each). The size stays what it was with one item per column
+// block, so that a workspace size, and which calls fit the allocation-free
+// entry's fixed one, does not depend on the tiling.
+size_t gemm_list_bytes(size_t M, size_t E, size_t N, bool gateup) {
+  const size_t cols = gateup ? 128 : 256;
+  return (4 + 4 * ((M + 255) / 256 + E) * ((N + cols - 1) / cols)) * 4;
+}
+
 Workspace layout(const moe_layer_desc* d, int T) {
   Workspace w{};
   const size_t A = 256, ds = dt_size(d->act_dtype);
@@ -495,7 +506,8 @@ Workspace layout(const moe_layer_desc* d, int T) {
   w.act = take(M * I * ds);
   w.Y = take(M * H * ds);
   w.plan_scratch = take(dispatch_scratch_bytes(T, (int)k, (int)E));
-  w.items = take(gemm_items_bytes((int)M, (int)E));
+  w.items = take(gemm_list_bytes(M, E, I, true));
+  take(gemm_list_bytes(M, E, H, false));
   w.x16 = take((size_t)T * H * 2);
   if (d->has_shared) {
     const size_t SI = (size_t)d->shared_up.n;
@@ -504,7 +516,8 @@ Workspace layout(const moe_layer_desc* d, int T) {
     w.s_act = take((size_t)T * SI * ds);
     w.s_out = take((size_t)T * H * ds);
     w.s_logit = take((size_t)T * ds);
-    w.s_items = take(gemm_items_bytes(T, 1));
+    w.s_items = take(gemm_list_bytes((size_t)T, 1, SI, true));
+    take(gemm_list_bytes((size_t)T, 1, H, false));
   }
   w.xn = take((size_t)T * H * ds);
   w.res = take((size_t)T * H * ds);
@@ -983,11 +996,16 @@ extern "C" moe_status moe_mxfp4_to_affine(const uint32_t* packed, const uint8_t*
   return ok();
 }
 
+size_t matmul_list_bytes(const moe_qproj* p, int M) {
+  return align_up(std::max(gemm_items_bytes(M, p->n_experts),
+                           gemm_list_bytes((size_t)M, (size_t)p->n_experts, (size_t)p->n, false)), 256);
+}
+
 // [used list / CSR copy][GEMM work list][bf16 rows as f16 operands]
 extern "C" size_t moe_expert_matmul_workspace_bytes(const moe_qproj* p, int32_t a_dtype, int32_t M) {
   if (!p || M <= 0 || validate_qproj_named(p, "expert_matmul") != MOE_OK || !dt_ok(a_dtype)) return 0;
   size_t bytes = align_up((size_t)(p->n_experts + 1) * 4, 256) +
-                 align_up(gemm_items_bytes(M, p->n_experts), 256);
+                 matmul_list_bytes(p, M);
   if (a_dtype == MOE_BF16) bytes += align_up((size_t)M * p->k * 2, 256);
   return bytes;
 }
@@ -1014,7 +1032,7 @@ extern "C" moe_status moe_expert_matmul(const moe_qproj* p, const void* a, int32
             "GEMM work list launch");
     const void* a16 = a;
     if (a_dtype == MOE_BF16) {  // the GEMM's f16 operand: bf16 rows scaled by 2^-kA16Shift
-      void* x16 = wsc + items_at + align_up(gemm_items_bytes(M, p->n_experts), 256);
+      void* x16 = wsc + items_at + matmul_list_bytes(p, M);
       const int64_t rows = perm ? (M + top_k - 1) / top_k : M;
       MOE_HIP(launch_to_a16(a, x16, rows * p->k, stream), "f16 operand launch");
       a16 = x16;
