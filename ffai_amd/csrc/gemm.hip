@@ -397,7 +397,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, const GemmLds L, ui
   // chunks of a segment: 2 at 32-value groups, else 4
   const bool g32 = a.gsh == 0;
   // tile j's pair of the lane's unit in a chunk (dead units of a half chunk
-  // take the last group's)
+  // read the last group's, which chunk_step masks)
   auto read_sb = [&](int chunk, bool tail, int j) -> h2_t {
     const int seg0 = g32 ? (chunk & ~1) : (chunk & ~3);
     int unit = 4 * (chunk - seg0) + kb;
@@ -475,6 +475,16 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, const GemmLds L, ui
       }
     }
     __builtin_amdgcn_sched_barrier(0);
+    // A half chunk's dead units get a zero scale and bias, and zero weights in
+    // the quarter at hand: the codes that follow the row, with the row's last
+    // scale, could overflow f16, and infinity times a masked activation is not zero.
+    if constexpr (LAST) {
+      const uint32_t live = tail && kb >= 2 ? 0u : ~0u;
+#pragma unroll
+      for (int j = 0; j < NT; j++)
+        q.v[j] = __builtin_bit_cast(h2_t, __builtin_bit_cast(uint32_t, q.v[j]) & live);
+      wa &= live;
+    }
     const WSet &cu = u[U % NSET], &nu = u[(U + 1) % NSET];
     u32x4_t wb;
 #pragma unroll

@@ -370,6 +370,45 @@ def test_expert_matmul_tile_edges(bits, dt, sb, gs, K, counts, N):
         check_close(got, ref, dt, f"tile edges bits={bits} gs={gs} K={K} rows={counts} N={N}")
 
 
+@pytest.mark.parametrize("bits", [2, 3, 4, 5, 6, 8])
+@pytest.mark.parametrize("dt", [BF16, F16])
+@pytest.mark.parametrize("K", [64, 192, 704])
+def test_expert_matmul_half_chunk_large_scales(bits, dt, K):
+    """K ends in half a chunk of the grouped GEMM. Each row's last group has a
+    scale whose product with its own small codes fits f16 and with the next
+    row's first codes (all ones) does not: what lies past a row's end takes no
+    part in its sums. Tolerance: the layer bar, as test_expert_matmul_mfma."""
+    rng = np.random.default_rng(bits * 100 + K)
+    E, N, gs, counts = 2, 24, 32, (40, 33)
+    top, G = 2 ** bits - 1, K // gs
+    codes = rng.integers(0, top + 1, (E, N, K)).astype(np.uint8)
+    codes[:, :, :32] = top
+    codes[:, :, -32:] = rng.integers(0, top // 2 + 1, (E, N, 32))
+    s = np.full((E, N, G), 1.0 / top)
+    s[:, :, -1] = 100000.0 / top
+    b = rng.uniform(-0.1, 0.1, (E, N, G))
+    w = np.stack([orc.pack_codes(codes[e], bits).reshape(N, K * bits // 32) for e in range(E)])
+    p = orc.QProj(w, store(s, F16), store(b, F16), bits, gs, F16)
+    M = int(sum(counts))
+    experts = np.repeat(np.arange(E), counts).astype(np.uint32)
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.uint32)
+    # f16: small enough for sums in f16's range; bf16 rows enter as f16 x 2^-8, normal numbers for these
+    a = store(rng.normal(0, 1.0 if dt == BF16 else 1e-3, (M, K)), dt)
+    lib = _lib.load()
+    q = _lib.QProj(0, 0, 0, None, bits, gs, F16, N, K, E)
+    wt, st, bt = to_torch(p.weight.view(np.int32)), to_torch(p.scales), to_torch(p.biases)
+    q.weight, q.scales, q.biases = wt.data_ptr(), st.data_ptr(), bt.data_ptr()
+    at = to_torch(a)
+    out = torch.empty(M, N, dtype=at.dtype, device="cuda")
+    wsb = lib.moe_expert_matmul_workspace_bytes(C.byref(q), dt, M)
+    ws = torch.empty(wsb, dtype=torch.uint8, device="cuda")
+    offt = to_torch(offsets.view(np.int32))
+    check(lib.moe_expert_matmul(C.byref(q), _p(at), dt, None, 1, M, _p(offt), _p(out), _p(ws), wsb, _stream()))
+    torch.cuda.synchronize()
+    ref = orc.round_dt(orc.qgemm_rows(p, load(a, dt), experts), dt)
+    check_close(to_numpy_f32(out), ref, dt, f"half chunk bits={bits} K={K}")
+
+
 @pytest.mark.parametrize("bits,dt,sb,gs,K", [
     (8, BF16, BF16, 64, 320),   # 8-bit codes as plain bf16 integers
     (8, BF16, F16, 32, 96),     # fewer units than a chunk
