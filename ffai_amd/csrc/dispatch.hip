@@ -259,6 +259,29 @@ hipError_t launch_route_plan(const void* logits, int dt, int T, int E, int k, co
   return hipErrorInvalidValue;
 }
 
+// The GEMM's row tiles of expert e, rows [off, off + n) of a sorted plan, by NT
+// threads (this one is t). Expert e's tiles start at slot off / kGemmTileRows + e,
+// which leaves room for every tile before them (ceil(c / R) <= floor((o + c) / R)
+// - floor(o / R) + 1), so no expert waits for a count of the others' tiles; a slot
+// without a tile holds no rows (kGemmNoTile). NT threads share an expert's tiles:
+// with one thread per expert, a single expert's list was a chain of stores that
+// grew with its rows (us of list and product at N 512, K 2048, 4 bits: 8192 rows
+// 48.1 -> 44.9, 32768 rows 139.9 -> 126.1).
+template <uint32_t NT>
+__device__ __forceinline__ void write_tiles(uint32_t e, uint32_t E, uint32_t off, uint32_t n, uint32_t t,
+                                            uint32_t* __restrict__ items) {
+  constexpr uint32_t R = kGemmTileRows;
+  const uint32_t first = off / R + e, end = (off + n) / R + e + 1u;
+  for (uint32_t i = t; i < end - first; i += NT) {
+    const uint32_t r = i * R;
+    const bool live = r < n;
+    items[4 + 2 * (first + i)] = live ? e : kGemmNoTile;
+    items[5 + 2 * (first + i)] = live ? (off + r) | ((min(n - r, R) - 1u) << 25) : 0u;
+  }
+  if (e == E - 1u && t == 0) items[0] = end;
+}
+static int item_blocks(int E) { return (E + kPlanThreads / 64 - 1) / (kPlanThreads / 64); }
+
 // The whole plan in one launch, a block per expert: every block reads all M ids
 // (held in registers, 4 QUADS per thread; 1024 threads, each wave a contiguous
 // share so that wave and lane order are token order), counts those below its
@@ -268,10 +291,7 @@ hipError_t launch_route_plan(const void* logits, int dt, int T, int E, int k, co
 // workgroup or three passes over chunks take (us: 1998 ids 11.8 -> 5.0, 4000
 // ids with the GEMM's row tiles 16.6 + 5.6 -> 5.5, 16384 ids on 256 experts
 // 5.3 + 5.5 + 9.8 -> 6.3, 32768 on 128 experts 4.9 + 4.9 + 10.6 -> 9.0).
-// items (nullable): also the GEMM's row tiles. Expert e's tiles start at slot
-// offset / kGemmTileRows + e, which leaves room for every tile before them
-// (ceil(c / R) <= floor((o + c) / R) - floor(o / R) + 1); a slot without a tile
-// holds no rows (kGemmNoTile).
+// items (nullable): also the GEMM's row tiles.
 // used (nullable): the used list, which needs the experts below e that occur:
 // a bitmap of them.
 template <int QUADS>
@@ -350,17 +370,7 @@ __global__ __launch_bounds__(1024) void plan_experts_kernel(
     offsets[e] = off;
     if (e == (uint32_t)E - 1u) offsets[E] = off + n;
   }
-  if (items) {
-    constexpr uint32_t R = kGemmTileRows;
-    const uint32_t first = off / R + e, end = (e == (uint32_t)E - 1u) ? (uint32_t)M / R + (uint32_t)E : (off + n) / R + e + 1u;
-    for (uint32_t t = (uint32_t)tid; t < end - first; t += 1024u) {
-      const uint32_t r = t * R;
-      const bool live = r < n;
-      items[4 + 2 * (first + t)] = live ? e : kGemmNoTile;
-      items[5 + 2 * (first + t)] = live ? (off + r) | ((min(n - r, R) - 1u) << 25) : 0u;
-    }
-    if (e == (uint32_t)E - 1u && tid == 0) items[0] = end;
-  }
+  if (items) write_tiles<1024>(e, (uint32_t)E, off, n, (uint32_t)tid, items);
   if (used) {
     __syncthreads();
     if (wave == 0) {
@@ -476,52 +486,26 @@ size_t dispatch_scratch_bytes(int T, int k, int E) {
   return (size_t)(nchunks * E * 4);
 }
 
-// Row tiles of the grouped GEMM over an expert-sorted plan (the list format is
-// described at launch_gemm_items): thread t counts the tiles of experts
-// t * EPT .. + EPT, a block scan gives each expert's first tile, and the
-// thread writes its experts' tiles (a tile holds up to kGemmTileRows rows, so
-// an expert has few).
-__device__ void gemm_items_body(const uint32_t* __restrict__ offsets, int E,
-                                uint32_t* __restrict__ items) {
-  __shared__ uint32_t wsum[kPlanThreads / 64];
-  constexpr int EPT = kPlanMaxE / kPlanThreads;  // experts per thread
-  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  uint32_t first[EPT], rows[EPT], tot = 0;
-#pragma unroll
-  for (int j = 0; j < EPT; j++) {
-    const int e = t * EPT + j;
-    first[j] = e < E ? offsets[e] : 0u;
-    rows[j] = e < E ? offsets[e + 1] - first[j] : 0u;
-    tot += (rows[j] + kGemmTileRows - 1u) / kGemmTileRows;
-  }
-  const uint32_t s = wave_scan_u32(tot);
-  if (lane == 63) wsum[wave] = s;
-  __syncthreads();
-  uint32_t at = s - tot, all = 0;
-#pragma unroll
-  for (int w = 0; w < kPlanThreads / 64; w++) {
-    at += w < wave ? wsum[w] : 0u;
-    all += wsum[w];
-  }
-  if (t == 0) items[0] = all;
-#pragma unroll
-  for (int j = 0; j < EPT; j++) {
-    for (uint32_t r = 0; r < rows[j]; r += kGemmTileRows, at++) {
-      items[4 + 2 * at] = (uint32_t)(t * EPT + j);
-      items[5 + 2 * at] = (first[j] + r) | ((min(rows[j] - r, (uint32_t)kGemmTileRows) - 1u) << 25);
-    }
-  }
+// The GEMM's row tiles from a plan's offsets: a wave per expert (waves before it
+// in a block of kPlanThreads and in `blk` blocks).
+__device__ __forceinline__ void gemm_items_body(const uint32_t* __restrict__ offsets, int E, int blk,
+                                                uint32_t* __restrict__ items) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int e = blk * (kPlanThreads / 64) + wave;
+  if (e >= E) return;
+  const uint32_t off = offsets[e];
+  write_tiles<64>((uint32_t)e, (uint32_t)E, off, offsets[e + 1] - off, threadIdx.x & 63u, items);
 }
 
 __global__ __launch_bounds__(kPlanThreads) void gemm_items_kernel(
     const uint32_t* __restrict__ offsets, int E, uint32_t* __restrict__ items) {
-  gemm_items_body(offsets, E, items);
+  gemm_items_body(offsets, E, (int)blockIdx.x, items);
 }
 
 // Multi-block pass 3 with the grouped GEMM's row tiles: each block scatters
-// its chunk as plan_scatter_kernel does, and one more block writes the tiles
-// (they need only the offsets, which the scan pass wrote). One launch fewer
-// per prefill step.
+// its chunk as plan_scatter_kernel does, and the blocks past the chunks write
+// the tiles (they need only the offsets, which the scan pass wrote). One launch
+// fewer per prefill step.
 __global__ __launch_bounds__(kPlanThreads) void plan_scatter_items_kernel(
     const uint32_t* __restrict__ idx, int M, int E, const uint32_t* __restrict__ hist,
     uint32_t* perm, uint32_t* inv, const uint32_t* __restrict__ offsets,
@@ -529,8 +513,9 @@ __global__ __launch_bounds__(kPlanThreads) void plan_scatter_items_kernel(
   __shared__ uint32_t cursor[kPlanMaxE];
   constexpr int PER = kChunk / kPlanThreads;
   const int tid = threadIdx.x, c = blockIdx.x;
-  if (c == (int)gridDim.x - 1) {
-    gemm_items_body(offsets, E, items);
+  const int nchunks = (M + kChunk - 1) / kChunk;
+  if (c >= nchunks) {  // block-uniform, before any barrier
+    gemm_items_body(offsets, E, c - nchunks, items);
     return;
   }
   const int begin = c * kChunk, end = min(M, begin + kChunk);
@@ -576,7 +561,7 @@ hipError_t launch_dispatch_plan(const uint32_t* idx, int T, int k, int E, uint32
   hipLaunchKernelGGL(plan_scan_kernel, dim3(1), dim3(kPlanThreads), 0, st, nchunks, E, hist,
                      counts, offsets, used);
   if (items) {
-    hipLaunchKernelGGL(plan_scatter_items_kernel, dim3(nchunks + 1), dim3(kPlanThreads), 0, st, idx,
+    hipLaunchKernelGGL(plan_scatter_items_kernel, dim3(nchunks + item_blocks(E)), dim3(kPlanThreads), 0, st, idx,
                        M, E, hist, perm, inv_perm, offsets, items);
     if (items_done) *items_done = true;
   } else {
@@ -588,7 +573,7 @@ hipError_t launch_dispatch_plan(const uint32_t* idx, int T, int k, int E, uint32
 
 hipError_t launch_gemm_items(const uint32_t* offsets, int E, uint32_t* items, hipStream_t st) {
   if (E > kPlanMaxE) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(gemm_items_kernel, dim3(1), dim3(kPlanThreads), 0, st, offsets, E, items);
+  hipLaunchKernelGGL(gemm_items_kernel, dim3(item_blocks(E)), dim3(kPlanThreads), 0, st, offsets, E, items);
   return hipGetLastError();
 }
 

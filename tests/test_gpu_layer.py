@@ -370,6 +370,32 @@ def test_expert_matmul_tile_edges(bits, dt, sb, gs, K, counts, N):
         check_close(got, ref, dt, f"tile edges bits={bits} gs={gs} K={K} rows={counts} N={N}")
 
 
+@pytest.mark.parametrize("counts", [(6300,), (1, 6145, 0, 0, 97, 0, 3000), (0, 0, 0, 6144)])
+def test_expert_matmul_many_tiles(counts):
+    """Experts with more row tiles than a wave has lanes (64 tiles of 96 rows
+    and one more, 64 exactly), alone and between experts without rows: every
+    row is written, once. Tolerance: the layer bar."""
+    from moe_spec import gen_qproj
+    rng = np.random.default_rng(sum(counts))
+    E, M, N, K, dt = len(counts), int(sum(counts)), 8, 64, BF16
+    p = gen_qproj(rng, E, N, K, 4, 64, BF16)
+    experts = np.repeat(np.arange(E), counts).astype(np.uint32)
+    a = store(rng.normal(0, 1, (M, K)), dt)
+    lib = _lib.load()
+    q = _lib.QProj(0, 0, 0, None, 4, 64, BF16, N, K, E)
+    wt, st, bt = to_torch(p.weight.view(np.int32)), to_torch(p.scales), to_torch(p.biases)
+    q.weight, q.scales, q.biases = wt.data_ptr(), st.data_ptr(), bt.data_ptr()
+    at = to_torch(a)
+    out = torch.full((M, N), float("nan"), dtype=at.dtype, device="cuda")
+    wsb = lib.moe_expert_matmul_workspace_bytes(C.byref(q), dt, M)
+    ws = torch.empty(wsb, dtype=torch.uint8, device="cuda")
+    offt = to_torch(np.concatenate([[0], np.cumsum(counts)]).astype(np.int32))
+    check(lib.moe_expert_matmul(C.byref(q), _p(at), dt, None, 1, M, _p(offt), _p(out), _p(ws), wsb, _stream()))
+    torch.cuda.synchronize()
+    ref = orc.round_dt(orc.qgemm_rows(p, load(a, dt), experts), dt)
+    check_close(to_numpy_f32(out), ref, dt, f"many tiles {counts}")
+
+
 @pytest.mark.parametrize("bits", [2, 3, 4, 5, 6, 8])
 @pytest.mark.parametrize("dt", [BF16, F16])
 @pytest.mark.parametrize("K", [64, 192, 704])
