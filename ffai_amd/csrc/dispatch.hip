@@ -11,9 +11,10 @@
 //      position = offsets[e] + (#earlier entries with expert e). The result is
 //      the stable order (expert asc, token asc, slot asc) bit for bit.
 //
-// Small plans run in one workgroup. Large plans (prefill) split the entries
-// into chunks: a per-chunk histogram pass, a scan pass, and a scatter pass
-// that starts every chunk at its own per-expert base.
+// Small plans run in one workgroup, most others in one launch of a block per
+// expert (plan_by_experts). The largest split the entries into chunks: a
+// per-chunk histogram pass, a scan pass, and a scatter pass that starts every
+// chunk at its own per-expert base.
 #include "moe_common.hpp"
 #include "moe_internal.hpp"
 
@@ -22,11 +23,28 @@ namespace moe {
 constexpr int kPlanThreads = 256;
 constexpr int kPlanMaxE = 1024;
 constexpr int kChunk = 1024;             // entries per chunk in the multi-block plan
-constexpr int kSingleBlockMax = 4096;    // M at or below which one workgroup plans
-// Entries for which a block per expert plans (plan_experts_kernel): up to the
-// ids 1024 threads hold in 32 registers each; from 512 entries one workgroup
-// (4.8 us there) takes longer than the 5 us it takes at any count up to 4096.
+constexpr int kSingleBlockMax = 1024;    // M at or below which one workgroup plans
+// Whether a block per expert plans (plan_experts_kernel) rather than one
+// workgroup (up to kSingleBlockMax entries) or the three passes over chunks. It
+// holds the ids of a block in 32 registers per thread at most, reads E M ids, and
+// one expert's entries are one block's to write, so it is kept to where it is the
+// faster one (us of the plan, the other way / a block per expert; 10 to 40 % less
+// with the GEMM's tiles in place of the used list):
+//  - above 512 entries: 513 on 128 experts 4.8 / 3.4; with more than 512 experts
+//    from 1024 (768 on 1024 experts 6.0 / 6.7, 1024 on 1024 7.0 / 6.7);
+//  - to 32768 entries on up to 256 experts (12.1 / 8.7), 16384 above (512 experts
+//    12.6 / 7.5, 1024 16.2 / 12.1; 32768 on 1024 20.8 / 28.3);
+//  - to 8192 entries per expert on average (8192 on one 8.8 / 6.0, 16384 on one
+//    8.9 / 10.1, 16384 on two 8.8 / 7.6, 32768 on two 9.7 / 13.3, on eight 10.3 /
+//    8.5). Uneven loads move the line only at the far end: half of 16384 entries
+//    on one of 128 experts 10.4 / 7.4, half of 32768 11.6 / 13.0.
 constexpr int kPlanExpertsMin = 512, kPlanExpertsMax = 32768;
+static bool plan_by_experts(int M, int E) {
+  if (M <= kPlanExpertsMin || M > kPlanExpertsMax) return false;
+  if (E > 512 && M < 1024) return false;
+  if (E > 256 && M > kPlanExpertsMax / 2) return false;
+  return M <= 8192 * E;
+}
 
 // Exclusive scan of cnt[0..E) over NT threads (4 experts per thread).
 // Writes offsets[0..E], counts, the used list, and base[e] = offsets[e].
@@ -292,15 +310,17 @@ static int item_blocks(int E) { return (E + kPlanThreads / 64 - 1) / (kPlanThrea
 // ids with the GEMM's row tiles 16.6 + 5.6 -> 5.5, 16384 ids on 256 experts
 // 5.3 + 5.5 + 9.8 -> 6.3, 32768 on 128 experts 4.9 + 4.9 + 10.6 -> 9.0).
 // items (nullable): also the GEMM's row tiles.
-// used (nullable): the used list, which needs the experts below e that occur:
-// a bitmap of them.
+// used (nullable): the used list, which needs how many experts below e occur: a
+// word per expert, set by plain stores (every store of a word writes the same
+// value). With atomics on a bitmap, lanes of one word took turns: 32768 ids on 32
+// experts 31.6 us, now 8.2; on 128 experts 14.9 -> 8.5.
 template <int QUADS>
 __global__ __launch_bounds__(1024) void plan_experts_kernel(
     const uint32_t* __restrict__ idx, int M, int E, uint32_t* __restrict__ counts,
     uint32_t* __restrict__ offsets, uint32_t* __restrict__ perm, uint32_t* __restrict__ inv,
     uint32_t* __restrict__ used, uint32_t* __restrict__ items) {
   __shared__ uint32_t wlt[16], weq[16];
-  __shared__ uint32_t seen[kPlanMaxE / 32];
+  __shared__ uint32_t seen[kPlanMaxE];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t e = blockIdx.x;
@@ -309,7 +329,7 @@ __global__ __launch_bounds__(1024) void plan_experts_kernel(
   u32x4_t id[QUADS];
 #pragma unroll
   for (int q = 0; q < QUADS; q++) id[q] = bload128(iv, (uint32_t)((wave * QUADS + q) * 64 + lane) * 16u);
-  if (used && tid < kPlanMaxE / 32) seen[tid] = 0;
+  if (used) seen[tid] = 0;  // kPlanMaxE threads
   uint32_t lt = 0, eq = 0;
 #pragma unroll
   for (int q = 0; q < QUADS; q++)
@@ -339,7 +359,7 @@ __global__ __launch_bounds__(1024) void plan_experts_kernel(
     for (int q = 0; q < QUADS; q++)
 #pragma unroll
       for (int c = 0; c < 4; c++)
-        if (id[q][c] < e) atomicOr(&seen[id[q][c] >> 5], 1u << (id[q][c] & 31u));
+        if (id[q][c] < e) seen[id[q][c]] = 1;
   }
   // this wave's entries of the expert, in order: quad by quad, lane by lane
   uint32_t run = off + at;
@@ -374,8 +394,9 @@ __global__ __launch_bounds__(1024) void plan_experts_kernel(
   if (used) {
     __syncthreads();
     if (wave == 0) {
-      const uint32_t w = lane < kPlanMaxE / 32 ? (uint32_t)__popc(seen[lane]) : 0u;
-      const uint32_t rank = (uint32_t)__builtin_amdgcn_readlane((int)wave_scan_u32(w), 63);
+      uint32_t rank = 0;
+#pragma unroll
+      for (int j = 0; j < kPlanMaxE / 64; j++) rank += (uint32_t)__popcll(__ballot(seen[64 * j + lane] != 0));
       if (lane == 0) {
         if (n) used[1 + rank] = e;
         if (e == (uint32_t)E - 1u) used[0] = rank + (n ? 1u : 0u);
@@ -481,7 +502,7 @@ __global__ __launch_bounds__(kPlanThreads) void used_from_offsets_kernel(const u
 
 size_t dispatch_scratch_bytes(int T, int k, int E) {
   const long M = (long)T * k;
-  if (M <= kSingleBlockMax) return 0;
+  if (M <= 4096) return 0;  // planned in one launch: the passes over chunks start above 8192
   const long nchunks = (M + kChunk - 1) / kChunk;
   return (size_t)(nchunks * E * 4);
 }
@@ -537,7 +558,7 @@ hipError_t launch_dispatch_plan(const uint32_t* idx, int T, int k, int E, uint32
   if (items_done) *items_done = false;
   const int M = T * k;
   if (E > kPlanMaxE) return hipErrorInvalidValue;
-  if (M > kPlanExpertsMin && M <= kPlanExpertsMax) {
+  if (plan_by_experts(M, E)) {
 #define MOE_PE(QUADS)                                                                              \
   hipLaunchKernelGGL((plan_experts_kernel<QUADS>), dim3(E), dim3(1024), 0, st, idx, M, E, counts,   \
                      offsets, perm, inv_perm, items ? nullptr : used, items)

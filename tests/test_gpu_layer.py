@@ -191,24 +191,33 @@ def test_layer_quantised_shared_gate(mixed, T):
     run_layer(with_quantised_router(mixed, bits=4, shared_gate_bits=4), T, seed=T + 1)
 
 
-@pytest.mark.parametrize("M,E", [(512, 16), (513, 5), (4096, 1), (4097, 300), (8193, 64), (16385, 1024),
-                                 (32768, 7), (32769, 40)])
-def test_dispatch_plan_edges(M, E):
-    """Entry counts around the plan's launch shapes (one workgroup, a block
-    per expert at 1, 2, 4 and 8 entries per thread and lane quad, the
-    chunked passes past 32768), k = 1, unused experts, and dropped ids."""
+@pytest.mark.parametrize("T,k,E", [
+    (512, 1, 16), (513, 1, 5), (4096, 1, 1), (4097, 1, 300), (8193, 1, 64), (16385, 1, 1024), (4096, 8, 7),
+    (32769, 1, 40),
+    (100, 8, 256), (171, 3, 1000), (682, 1, 700),  # the used list past 512 entries; one workgroup above 512 experts
+    (1023, 1, 1024), (1024, 1, 1024), (16384, 1, 1024), (16388, 1, 300),  # limits of the block-per-expert plan
+    (8192, 1, 1), (8193, 1, 1), (8192, 2, 2), (16385, 1, 2), (5461, 6, 256), (5462, 6, 257),
+])
+def test_dispatch_plan_edges(T, k, E):
+    """Entry, expert and token counts around the plan's launch shapes (one
+    workgroup, a block per expert at 1, 2, 4 and 8 entries per thread and lane
+    quad, the passes over chunks), unused experts and dropped ids. The used
+    list is the workspace's first words."""
+    M = T * k
     rng = np.random.default_rng(M + E)
     idx = rng.integers(0, E, M).astype(np.uint32)
     if E > 4:
         idx[idx == 3] = 2                # an expert without entries
+    if E > 200:
+        idx[(idx > 64) & (idx < 130)] = 130
     idx[rng.random(M) < 0.02] = E + 5    # out of range: dropped
     lib = _lib.load()
     out = {n: torch.full((sz,), -1, dtype=torch.int32, device="cuda")
            for n, sz in (("counts", E), ("offsets", E + 1), ("perm", M), ("inv", M))}
-    wsb = lib.moe_dispatch_workspace_bytes(M, 1, E)
-    ws = torch.empty(max(wsb, 1), dtype=torch.uint8, device="cuda")
+    wsb = lib.moe_dispatch_workspace_bytes(T, k, E)
+    ws = torch.full((max(wsb, 4) // 4,), -1, dtype=torch.int32, device="cuda")
     idxt = to_torch(idx.view(np.int32))
-    check(lib.moe_dispatch_plan(_p(idxt), M, 1, E, _p(out["counts"]), _p(out["offsets"]), _p(out["perm"]),
+    check(lib.moe_dispatch_plan(_p(idxt), T, k, E, _p(out["counts"]), _p(out["offsets"]), _p(out["perm"]),
                                 _p(out["inv"]), _p(ws), wsb, _stream()))
     torch.cuda.synchronize()
     kept = np.nonzero(idx < E)[0]
@@ -220,6 +229,9 @@ def test_dispatch_plan_edges(M, E):
     inv = _u32(out["inv"])
     assert np.array_equal(inv[order], np.arange(len(order)))
     assert np.all(inv[idx >= E] == 0xFFFFFFFF)  # left unwritten
+    used = _u32(ws)[:E + 1]
+    assert used[0] == np.count_nonzero(counts)
+    assert np.array_equal(used[1:1 + used[0]], np.nonzero(counts)[0])
 
 
 @pytest.mark.parametrize("T,k,E", [(1, 8, 128), (1, 4, 32), (16, 2, 8), (64, 8, 128), (512, 8, 128),
