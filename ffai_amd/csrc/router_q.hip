@@ -76,8 +76,11 @@ __global__ __launch_bounds__(256) void router_qrow_kernel(const XT* __restrict__
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 // Tiles of a launch below which a tile's hidden dimension goes over 16 waves
 // instead of 4: with few blocks the launch lasts as long as one wave's chain of
-// chunks (48 tokens, 64 experts of hidden 1024 at 8 bits, 16 chunks: 9.9 ->
-// 7.5 us).
+// chunks. 48 tokens, 64 experts, us with 4 / 16 waves: hidden 512 at 8 bits 5.5 /
+// 4.4, 1024 8.7 / 7.3, 2048 14.0 / 13.3, 2880 12.1 / 11.5, 4096 24.2 / 23.8, 7168
+// 39.6 / 38.2. (While loads past a wave's last
+// chunk repeated that chunk, 16 waves lost from two chunks a wave on: 2048 at 8
+// bits 13.9 / 16.9, 4096 24.3 / 27.3.)
 constexpr int kRqFewTiles = 256;
 
 template <typename XT> struct RqMfma;
@@ -164,7 +167,7 @@ __global__ __launch_bounds__(64 * NW) void router_qgemm_kernel(const XT* __restr
   const uint32_t wo = ex * (uint32_t)row_words * 4u;
   const uint32_t so = ex * (uint32_t)groups;
   const int G = H >> 6;
-  const int ng = (G - wv + NW - 1) / NW;  // chunks wv + 4 i, i < ng
+  const int ng = (G - wv + NW - 1) / NW;  // chunks wv + NW i, i < ng
 
   struct Set {
     u32x4_t a[4];
@@ -172,15 +175,18 @@ __global__ __launch_bounds__(64 * NW) void router_qgemm_kernel(const XT* __restr
     ST s[2], b[2];
   };
   auto load = [&](int i, Set& st) __attribute__((always_inline)) {
-    const int c = min(wv + NW * i, G - 1);  // clamped: in bounds, never multiplied
-    const uint32_t kb = (uint32_t)c * 128u;
+    const int c0 = wv + NW * i, c = min(c0, G - 1);  // clamped: in bounds, never multiplied
+    // With 16 waves a load past a wave's last chunk is a large part of its few
+    // loads: offset past the views (scalar), it reads nothing.
+    const uint32_t dead = NW > 4 && c0 >= G ? 0x80000000u : 0u;
+    const uint32_t kb = (uint32_t)c * 128u + dead;
 #pragma unroll
     for (int q = 0; q < 4; q++) st.a[q] = bload128(xr, xo + kb + 32u * (uint32_t)q);
 #pragma unroll
     for (int u = 0; u < 2; u++) {
       const int unit = 2 * c + u;
-      bload_unit<BITS>(wr, wo + (uint32_t)(unit * BITS) * 4u, st.w[u]);
-      const uint32_t gi = (so + (uint32_t)(unit >> gsh)) * (uint32_t)sizeof(ST);
+      bload_unit<BITS>(wr, wo + ((uint32_t)(unit * BITS) * 4u + dead), st.w[u]);
+      const uint32_t gi = (so + (uint32_t)(unit >> gsh)) * (uint32_t)sizeof(ST) + dead;
       st.s[u] = __builtin_bit_cast(ST, bload16(sr, gi));
       st.b[u] = __builtin_bit_cast(ST, bload16(br, gi));
     }

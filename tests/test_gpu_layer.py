@@ -135,8 +135,11 @@ def test_router_logits_within_one_ulp(dt, wdt, E, H, T):
     (7, 40, 1024, 32, F16, False),     # a few tokens, E not a multiple of 32
     (64, 128, 2048, 64, BF16, False),  # many tokens: the matrix-core kernel
     (96, 64, 768, 128, F16, True),
-    (40, 40, 512, 64, BF16, True),     # many tokens, E % 32 != 0: the row kernel
+    (40, 40, 512, 64, BF16, True),     # E % 32 != 0
     (2016, 128, 128, 64, BF16, False), # 252 tiles: 16 waves per tile, 2 chunks
+    (64, 64, 2880, 64, BF16, True),    # 16 waves of 3 or 2 chunks
+    (33, 65, 3072, 64, F16, False),    # 16 waves of 3 chunks
+    (32, 32, 1088, 64, BF16, False),   # 16 waves of 2 or 1
     # 256 tiles: 4 waves per tile (no bias: the bound is two ulps of the logit
     # itself, and among 2^18 logits a bias cancels some product of magnitude 2 to
     # 4, whose own f16 ulp is 2^-9 to 2^-8, down to a far smaller logit)
