@@ -574,7 +574,9 @@ constexpr int kMmaMinRowsSingleExpert10 = 160;
 // activation rows per pass instead of 16 (µs per layer step, 16 / 32 rows per
 // pass: 15.6 rows on 128 experts 342 / 327, 16 and 23 rows on 32 large experts
 // 226 / 199 and 276 / 225; at 10 and 14 rows on 128 experts 126 / 150 and
-// 150 / 155).
+// 150 / 155). Only where one expert can have more than 16 rows, which a narrow
+// pass holds (16 rows of one expert of 2048 x 2048: 12.7 / 15.1; 17 rows 19.7 /
+// 15.1).
 constexpr int kMmaWideRows10 = 150;
 
 // gemv_mma_kernel applies: codes of one width (every width is exact in either
@@ -677,8 +679,8 @@ void run_multi(const moe_qproj& p0, const moe_qproj* p1, const void* x, int xdt,
 // block, 16 activation rows per pass. The caller has checked mma_ok.
 void run_mma(const moe_qproj& p0, const moe_qproj* p1, const void* x, int xdt,
              const uint32_t* perm, int topk, const uint32_t* offsets, const uint32_t* used, int slots,
-             int M, int x_rows, void* out, int act, float alpha, float limit, hipStream_t st, KEvents ev,
-             moe_status* status) {
+             int M, int max_rows, int x_rows, void* out, int act, float alpha, float limit, hipStream_t st,
+             KEvents ev, moe_status* status) {
   const int rows_per_block = p1 ? 32 : 64;
   const int row_blocks = (p0.n + rows_per_block - 1) / rows_per_block;
   GemvArgs a{};
@@ -699,7 +701,7 @@ void run_mma(const moe_qproj& p0, const moe_qproj* p1, const void* x, int xdt,
   a.alpha = alpha;
   a.limit = limit;
   a.x_rows = x_rows;
-  a.tok_chunk = 10L * M >= (long)kMmaWideRows10 * std::max(1, slots) ? 32 : 16;
+  a.tok_chunk = max_rows > 16 && 10L * M >= (long)kMmaWideRows10 * std::max(1, slots) ? 32 : 16;
   *status = hip_check(launch_mma(p0.bits, xdt, p0.sb_dtype, p1 != nullptr, a, slots * row_blocks, st, ev),
                       "grouped GEMV launch");
 }
@@ -716,7 +718,7 @@ moe_status run_gemv(const moe_qproj& p0, const moe_qproj* p1, const void* x, int
     moe_status status = MOE_OK;
     // the activation rows: one per token on the gather path (M = T topk)
     const int x_rows = perm ? (M + topk - 1) / topk : M;
-    run_mma(p0, p1, x, xdt, perm, topk, offsets, used, slots, M, x_rows, out, act, alpha, limit, st,
+    run_mma(p0, p1, x, xdt, perm, topk, offsets, used, slots, M, std::min(max_rows, M), x_rows, out, act, alpha, limit, st,
             ev, &status);
     return status;
   }

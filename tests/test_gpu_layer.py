@@ -460,7 +460,7 @@ def test_expert_matmul_half_chunk_large_scales(bits, dt, K):
     (3, BF16, BF16, 64, 576),
     (6, BF16, F16, 32, 288),
 ])
-@pytest.mark.parametrize("counts", [(2, 5, 1), (16, 1, 17), (17, 33, 16), (0, 32, 31)])
+@pytest.mark.parametrize("counts", [(2, 5, 1), (16, 1, 17), (17, 33, 16), (0, 32, 31), (16,), (17,)])
 @pytest.mark.parametrize("N", [24, 65])
 def test_expert_matmul_mma_gemv(bits, dt, sb, gs, K, counts, N):
     """The batched matrix-core GEMV at one row, a full and an overfull pass of
