@@ -102,6 +102,12 @@ hipError_t launch_gemm_b4(int, bool, const GemmArgs&, int, hipStream_t, KEvents)
 hipError_t launch_gemm_b5(int, bool, const GemmArgs&, int, hipStream_t, KEvents);
 hipError_t launch_gemm_b6(int, bool, const GemmArgs&, int, hipStream_t, KEvents);
 hipError_t launch_gemm_b8(int, bool, const GemmArgs&, int, hipStream_t, KEvents);
+hipError_t launch_gemm_tall_b2(int, bool, const GemmArgs&, int, hipStream_t, KEvents);
+hipError_t launch_gemm_tall_b3(int, bool, const GemmArgs&, int, hipStream_t, KEvents);
+hipError_t launch_gemm_tall_b4(int, bool, const GemmArgs&, int, hipStream_t, KEvents);
+hipError_t launch_gemm_tall_b5(int, bool, const GemmArgs&, int, hipStream_t, KEvents);
+hipError_t launch_gemm_tall_b6(int, bool, const GemmArgs&, int, hipStream_t, KEvents);
+hipError_t launch_gemm_tall_b8(int, bool, const GemmArgs&, int, hipStream_t, KEvents);
 
 hipError_t launch_gemm(int bits, int xdt, int sbdt, bool gateup, const GemmArgs& a0, int grid,
                        hipStream_t st, KEvents ev) {
@@ -109,12 +115,12 @@ hipError_t launch_gemm(int bits, int xdt, int sbdt, bool gateup, const GemmArgs&
   GemmArgs a = a0;
   a.sb_bf16 = sbdt == DT_BF16;
   switch (bits) {
-    case 2: return launch_gemm_b2(xdt, gateup, a, grid, st, ev);
-    case 3: return launch_gemm_b3(xdt, gateup, a, grid, st, ev);
-    case 4: return launch_gemm_b4(xdt, gateup, a, grid, st, ev);
-    case 5: return launch_gemm_b5(xdt, gateup, a, grid, st, ev);
-    case 6: return launch_gemm_b6(xdt, gateup, a, grid, st, ev);
-    case 8: return launch_gemm_b8(xdt, gateup, a, grid, st, ev);
+    case 2: return (a.tall ? launch_gemm_tall_b2 : launch_gemm_b2)(xdt, gateup, a, grid, st, ev);
+    case 3: return (a.tall ? launch_gemm_tall_b3 : launch_gemm_b3)(xdt, gateup, a, grid, st, ev);
+    case 4: return (a.tall ? launch_gemm_tall_b4 : launch_gemm_b4)(xdt, gateup, a, grid, st, ev);
+    case 5: return (a.tall ? launch_gemm_tall_b5 : launch_gemm_b5)(xdt, gateup, a, grid, st, ev);
+    case 6: return (a.tall ? launch_gemm_tall_b6 : launch_gemm_b6)(xdt, gateup, a, grid, st, ev);
+    case 8: return (a.tall ? launch_gemm_tall_b8 : launch_gemm_b8)(xdt, gateup, a, grid, st, ev);
   }
   return hipErrorInvalidValue;
 }
@@ -795,11 +801,34 @@ bool gemm_ok(const moe_qproj& p, int xdt, int M, const void* out = nullptr) {
          (reinterpret_cast<uintptr_t>(out) & 15) == 0;
 }
 
-// out[p] = W[e(p)] . a[row(p)] (or the gate/up pair with the activation)
-// over a plan, on the matrix cores. `items` must hold the work list written by
-// launch_gemm_items for the same offsets and (N, gate/up). The A rows x are
-// f16 A operands (kA16Shift); a gate/up pair writes its activation as A
-// rows.
+// Whether a GEMM call of M rows takes the tall kernel's 256-row tiles. From some
+// average of rows per expert on, its one dequantisation of a weight per 256 rows
+// outweighs the small blocks' better overlap, sooner the more a code costs to
+// unpack (us per layer step, small blocks / tall): 32 experts of 2880 x 2880,
+//   4 bits: 256 rows 598 / 623, 320 rows 716 / 724, 384 rows 827 / 793, 512 rows
+//     1059 / 1015, 1024 rows 2006 / 1802; uneven loads, 375 rows 831 / 769;
+//   6 bits: 137 rows 462 / 466, 192 rows 582 / 540, 512 rows 1242 / 1130;
+//   8 bits: 96 rows 434 / 424, 112 rows 477 / 443, 256 rows 768 / 680, 512 rows
+//     1343 / 1113;
+// 128 experts of 2048 x 768, 4 bits: 287 rows 515 / 547, 384 rows 667 / 635, 512
+// rows 852 / 817. Even loads of 170 to 205 rows at up to 5 bits fit one 256-row
+// tile, where tall tiles are up to 7 % faster, but uneven ones of that average are
+// up to 7 % slower (192 rows 478 / 450 and 476 / 511), so the line stays above.
+// Few blocks fill few rounds over the CUs with one block each (under
+// kTallMinBlocks: 8 bits, 64 experts of 1024 x 384, 2048 tokens 114 / 125, 4096
+// tokens 184 / 166; 4 bits, 32 experts of 2048 x 1024, 3200 tokens 246 / 276), and
+// few chunks of K leave prologue and epilogue in the open (64 experts of 1024 x
+// 384, 1024 rows 273 / 292; at 8 bits 64 experts of 1024 x 1024, 512 rows 365 / 340).
+constexpr long kTallMinBlocks = 700;
+bool gemm_tall(const moe_qproj& p, bool pair, int M) {
+  const long slots = std::min(p.n_experts, M);
+  const long min_rows = p.bits <= 5 ? 325 : p.bits == 6 ? 190 : 110;
+  const int min_k = p.bits == 8 ? 1024 : 2048;
+  const long tiles = slots * ((M / slots + kTallTileRows - 1) / kTallTileRows);
+  return p.k >= min_k && M >= min_rows * slots && M <= (1 << kTallRowShift) &&
+         tiles * gemm_col_blocks(p.n, pair, true) >= kTallMinBlocks;
+}
+
 // The routed experts / the shared expert of a layer call of T rows take the
 // grouped GEMM (gate/up and down together: the gate/up epilogue writes the
 // down GEMM's f16 operand).
@@ -816,10 +845,14 @@ bool shared_gemm(const moe_layer_desc* d, int T) {
          (d->activation == MOE_ACT_RELU2 || sb_words_ok(d->shared_up));
 }
 
+// out[p] = W[e(p)] . a[row(p)] (or the gate/up pair with the activation)
+// over a plan, on the matrix cores. `items` must hold the row tiles written by
+// the plan or launch_gemm_items for the same offsets and `tall`. The A rows x are
+// f16 A operands (kA16Shift); a gate/up pair writes its activation as A rows.
 // out_a16: a single projection writes A rows for a following GEMM (the
 // first stage of squared-ReLU experts).
-moe_status run_gemm(const moe_qproj& p0, const moe_qproj* p1, const void* x, int xdt, bool out_a16, const uint32_t* perm, int topk, const uint32_t* offsets,
-                    const uint32_t* items, int M, void* out, int act, float alpha, float limit,
+moe_status run_gemm(const moe_qproj& p0, const moe_qproj* p1, const void* x, int xdt, bool out_a16,
+                    const uint32_t* perm, int topk, const uint32_t* items, bool tall, int M, void* out, int act, float alpha, float limit,
                     hipStream_t st, KEvents ev = {}) {
   GemmArgs a{};
   a.out_a16 = out_a16;
@@ -829,7 +862,6 @@ moe_status run_gemm(const moe_qproj& p0, const moe_qproj* p1, const void* x, int
   a.x_rows = perm ? (M + topk - 1) / topk : M;
   a.perm = perm;
   a.topk = topk;
-  a.offsets = offsets;
   a.items = items;
   a.out = out;
   a.N = p0.n;
@@ -839,8 +871,9 @@ moe_status run_gemm(const moe_qproj& p0, const moe_qproj* p1, const void* x, int
   a.alpha = alpha;
   a.limit = limit;
   const bool gu = p1 != nullptr;
-  a.col_blocks = gemm_col_blocks(p0.n, gu);
-  const long most = gemm_max_tiles(M, p0.n_experts) * a.col_blocks;
+  a.tall = tall;
+  a.col_blocks = gemm_col_blocks(p0.n, gu, tall);
+  const long most = gemm_max_tiles(M, p0.n_experts, tall) * a.col_blocks;
   const int grid = (int)((most + 7) / 8 * 8);  // a multiple of the 8 XCDs
   MOE_HIP(launch_gemm(p0.bits, xdt, p0.sb_dtype, gu, a, grid, st, ev),
           "grouped GEMM launch");
@@ -1030,7 +1063,8 @@ extern "C" moe_status moe_expert_matmul(const moe_qproj* p, const void* a, int32
     char* wsc = reinterpret_cast<char*>(workspace);
     const size_t items_at = align_up((size_t)(p->n_experts + 1) * 4, 256);
     uint32_t* items = reinterpret_cast<uint32_t*>(wsc + items_at);
-    MOE_HIP(launch_gemm_items(offsets, p->n_experts, items, stream),
+    const bool tall = gemm_tall(*p, false, M);
+    MOE_HIP(launch_gemm_items(offsets, p->n_experts, items, tall, stream),
             "GEMM work list launch");
     const void* a16 = a;
     if (a_dtype == MOE_BF16) {  // the GEMM's f16 operand: bf16 rows scaled by 2^-kA16Shift
@@ -1039,7 +1073,7 @@ extern "C" moe_status moe_expert_matmul(const moe_qproj* p, const void* a, int32
       MOE_HIP(launch_to_a16(a, x16, rows * p->k, stream), "f16 operand launch");
       a16 = x16;
     }
-    MOE_TRY(run_gemm(*p, nullptr, a16, a_dtype, false, perm, top_k, offsets, items, M, out, 0, 0.f,
+    MOE_TRY(run_gemm(*p, nullptr, a16, a_dtype, false, perm, top_k, items, tall, M, out, 0, 0.f,
                      0.f, stream));
     return ok();
   }
@@ -1265,13 +1299,13 @@ moe_status shared_expert(const moe_layer_desc* d, const void* x, const void* x16
   const moe_qproj* p1 = gated ? &d->shared_up : nullptr;
   if (shared_gemm(d, T)) {
     // many tokens through one expert: the matrix-core path
-    MOE_HIP(launch_gemm_items(at<uint32_t>(ws, w.s_off), 1, at<uint32_t>(ws, w.s_items), st),
+    MOE_HIP(launch_gemm_items(at<uint32_t>(ws, w.s_off), 1, at<uint32_t>(ws, w.s_items), false, st),
             "shared GEMM work list launch");
-    MOE_TRY(run_gemm(p0, p1, x16, xdt, true, nullptr, 1, at<uint32_t>(ws, w.s_off),
-                     at<uint32_t>(ws, w.s_items), T, at<void>(ws, w.s_act), d->activation,
+    MOE_TRY(run_gemm(p0, p1, x16, xdt, true, nullptr, 1,
+                     at<uint32_t>(ws, w.s_items), false, T, at<void>(ws, w.s_act), d->activation,
                      d->act_alpha, d->act_limit, st));
     MOE_TRY(run_gemm(d->shared_down, nullptr, at<void>(ws, w.s_act), xdt, false, nullptr, 1,
-                     at<uint32_t>(ws, w.s_off), at<uint32_t>(ws, w.s_items), T,
+                     at<uint32_t>(ws, w.s_items), false, T,
                      at<void>(ws, w.s_out), 0, 0.f, 0.f, st));
   } else {
     MOE_TRY(run_gemv(p0, p1, x, xdt, nullptr, 1, at<uint32_t>(ws, w.s_off),
@@ -1613,7 +1647,7 @@ moe_status layer_forward(const moe_layer_desc* d, const void* x, const void* rx,
                                    at<uint32_t>(ws, w.offsets), at<uint32_t>(ws, w.perm),
                                    at<uint32_t>(ws, w.inv), at<uint32_t>(ws, w.used),
                                    at<void>(ws, w.plan_scratch), dispatch_scratch_bytes(T, k, E),
-                                   st, nullptr, nullptr),
+                                   st),
               "dispatch plan launch");
     MOE_TRY(side.join());
     if (smode)
@@ -1625,7 +1659,9 @@ moe_status layer_forward(const moe_layer_desc* d, const void* x, const void* rx,
     const bool gated = d->activation != MOE_ACT_RELU2;
     const moe_qproj& p0 = gated ? d->gate : d->up;
     const moe_qproj* p1 = gated ? &d->up : nullptr;
-    // the GEMM's row tiles, written by the plan's last launch when it can
+    // the GEMM's row tiles (of one height for both its launches), written by the
+    // plan's last launch when it can
+    const bool tall = gemm && gemm_tall(p0, p1 != nullptr, M);
     bool items_done = false;
     // 2. selection + dispatch plan (MoELayer.swift:706-792): one launch for a
     //    small batch, else the top-k and plan kernels (past 8 tokens the GEMM
@@ -1645,17 +1681,17 @@ moe_status layer_forward(const moe_layer_desc* d, const void* x, const void* rx,
                                    at<uint32_t>(ws, w.offsets), at<uint32_t>(ws, w.perm),
                                    at<uint32_t>(ws, w.inv), at<uint32_t>(ws, w.used),
                                    at<void>(ws, w.plan_scratch), dispatch_scratch_bytes(T, k, E),
-                                   st, gemm ? at<uint32_t>(ws, w.items) : nullptr, &items_done),
+                                   st, gemm ? at<uint32_t>(ws, w.items) : nullptr, tall, &items_done),
               "dispatch plan launch");
     }
     const int slots = std::min(E, M);
     // 3. gate/up + activation over the plan (MoELayer.swift:883-893)
     if (gemm) {
       if (!items_done)
-        MOE_HIP(launch_gemm_items(at<uint32_t>(ws, w.offsets), E, at<uint32_t>(ws, w.items), st),
+        MOE_HIP(launch_gemm_items(at<uint32_t>(ws, w.offsets), E, at<uint32_t>(ws, w.items), tall, st),
                 "GEMM work list launch");
       MOE_TRY(run_gemm(p0, p1, x16, xdt, true, at<uint32_t>(ws, w.perm), k,
-                       at<uint32_t>(ws, w.offsets), at<uint32_t>(ws, w.items), M,
+                       at<uint32_t>(ws, w.items), tall, M,
                        at<void>(ws, w.act), d->activation, d->act_alpha, d->act_limit, st, kev(0)));
     } else {
       MOE_TRY(run_gemv(p0, p1, x, xdt, at<uint32_t>(ws, w.perm), k,
@@ -1666,7 +1702,7 @@ moe_status layer_forward(const moe_layer_desc* d, const void* x, const void* rx,
     // 4. down projection, then the weighted combine (MoELayer.swift:899-939)
     if (gemm) {
       MOE_TRY(run_gemm(d->down, nullptr, at<void>(ws, w.act), xdt, false, nullptr, 1,
-                       at<uint32_t>(ws, w.offsets), at<uint32_t>(ws, w.items), M,
+                       at<uint32_t>(ws, w.items), tall, M,
                        at<void>(ws, w.Y), 0, 0.f, 0.f, st, kev(1)));
     } else {
       MOE_TRY(run_gemv(d->down, nullptr, at<void>(ws, w.act), xdt, nullptr, 1,

@@ -15,6 +15,8 @@
 // expert (plan_by_experts). The largest split the entries into chunks: a
 // per-chunk histogram pass, a scan pass, and a scatter pass that starts every
 // chunk at its own per-expert base.
+#include <algorithm>
+
 #include "moe_common.hpp"
 #include "moe_internal.hpp"
 
@@ -277,29 +279,6 @@ hipError_t launch_route_plan(const void* logits, int dt, int T, int E, int k, co
   return hipErrorInvalidValue;
 }
 
-// The GEMM's row tiles of expert e, rows [off, off + n) of a sorted plan, by NT
-// threads (this one is t). Expert e's tiles start at slot off / kGemmTileRows + e,
-// which leaves room for every tile before them (ceil(c / R) <= floor((o + c) / R)
-// - floor(o / R) + 1), so no expert waits for a count of the others' tiles; a slot
-// without a tile holds no rows (kGemmNoTile). NT threads share an expert's tiles:
-// with one thread per expert, a single expert's list was a chain of stores that
-// grew with its rows (us of list and product at N 512, K 2048, 4 bits: 8192 rows
-// 48.1 -> 44.9, 32768 rows 139.9 -> 126.1).
-template <uint32_t NT>
-__device__ __forceinline__ void write_tiles(uint32_t e, uint32_t E, uint32_t off, uint32_t n, uint32_t t,
-                                            uint32_t* __restrict__ items) {
-  constexpr uint32_t R = kGemmTileRows;
-  const uint32_t first = off / R + e, end = (off + n) / R + e + 1u;
-  for (uint32_t i = t; i < end - first; i += NT) {
-    const uint32_t r = i * R;
-    const bool live = r < n;
-    items[4 + 2 * (first + i)] = live ? e : kGemmNoTile;
-    items[5 + 2 * (first + i)] = live ? (off + r) | ((min(n - r, R) - 1u) << 25) : 0u;
-  }
-  if (e == E - 1u && t == 0) items[0] = end;
-}
-static int item_blocks(int E) { return (E + kPlanThreads / 64 - 1) / (kPlanThreads / 64); }
-
 // The whole plan in one launch, a block per expert: every block reads all M ids
 // (held in registers, 4 QUADS per thread; 1024 threads, each wave a contiguous
 // share so that wave and lane order are token order), counts those below its
@@ -309,7 +288,10 @@ static int item_blocks(int E) { return (E + kPlanThreads / 64 - 1) / (kPlanThrea
 // workgroup or three passes over chunks take (us: 1998 ids 11.8 -> 5.0, 4000
 // ids with the GEMM's row tiles 16.6 + 5.6 -> 5.5, 16384 ids on 256 experts
 // 5.3 + 5.5 + 9.8 -> 6.3, 32768 on 128 experts 4.9 + 4.9 + 10.6 -> 9.0).
-// items (nullable): also the GEMM's row tiles.
+// items (nullable): also the GEMM's row tiles. Expert e's tiles start at slot
+// offset / kGemmTileRows + e, which leaves room for every tile before them
+// (ceil(c / R) <= floor((o + c) / R) - floor(o / R) + 1); a slot without a tile
+// holds no rows (kGemmNoTile).
 // used (nullable): the used list, which needs how many experts below e occur: a
 // word per expert, set by plain stores (every store of a word writes the same
 // value). With atomics on a bitmap, lanes of one word took turns: 32768 ids on 32
@@ -390,7 +372,17 @@ __global__ __launch_bounds__(1024) void plan_experts_kernel(
     offsets[e] = off;
     if (e == (uint32_t)E - 1u) offsets[E] = off + n;
   }
-  if (items) write_tiles<1024>(e, (uint32_t)E, off, n, (uint32_t)tid, items);
+  if (items) {
+    constexpr uint32_t R = kGemmTileRows;
+    const uint32_t first = off / R + e, end = (off + n) / R + e + 1u;
+    for (uint32_t t = (uint32_t)tid; t < end - first; t += 1024u) {
+      const uint32_t r = t * R;
+      const bool live = r < n;
+      items[4 + 2 * (first + t)] = live ? e : kGemmNoTile;
+      items[5 + 2 * (first + t)] = live ? (off + r) | ((min(n - r, R) - 1u) << kGemmRowShift) : 0u;
+    }
+    if (e == (uint32_t)E - 1u && tid == 0) items[0] = end;
+  }
   if (used) {
     __syncthreads();
     if (wave == 0) {
@@ -507,20 +499,64 @@ size_t dispatch_scratch_bytes(int T, int k, int E) {
   return (size_t)(nchunks * E * 4);
 }
 
-// The GEMM's row tiles from a plan's offsets: a wave per expert (waves before it
-// in a block of kPlanThreads and in `blk` blocks).
-__device__ __forceinline__ void gemm_items_body(const uint32_t* __restrict__ offsets, int E, int blk,
-                                                uint32_t* __restrict__ items) {
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int e = blk * (kPlanThreads / 64) + wave;
-  if (e >= E) return;
-  const uint32_t off = offsets[e];
-  write_tiles<64>((uint32_t)e, (uint32_t)E, off, offsets[e + 1] - off, threadIdx.x & 63u, items);
+// Row tiles of the grouped GEMM over an expert-sorted plan (the list format is
+// described at launch_gemm_items), by block `blk` of `nblk`: every block counts
+// each expert's tiles and scans the counts for its first one (thread t: experts
+// t * EPT .. + EPT), then a wave per expert writes its tiles. With one thread per
+// expert, a single expert's list was a chain of stores that grew with its rows (us
+// of list and product at N 512, K 2048, 4 bits: 8192 rows 48.1 -> 44.9, 32768
+// rows 139.9 -> 126.1). Without the scan, each expert from a slot its offset
+// gives, the list's empty slots leave the XCDs with unequal shares of the tiles:
+// for 256-row tiles up to a tenth of a layer step (8-bit, 32 experts of 2880 x
+// 2880, 1800 tokens 655 -> 596).
+__device__ __forceinline__ void gemm_items_body(const uint32_t* __restrict__ offsets, int E, int blk, int nblk,
+                                                bool tall, uint32_t* __restrict__ items) {
+  __shared__ uint32_t wsum[kPlanThreads / 64], start[kPlanMaxE];
+  constexpr int EPT = kPlanMaxE / kPlanThreads;  // experts per thread
+  const uint32_t R = tall ? kTallTileRows : kGemmTileRows;
+  const int shift = tall ? kTallRowShift : kGemmRowShift;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  uint32_t tiles[EPT], tot = 0;
+#pragma unroll
+  for (int j = 0; j < EPT; j++) {
+    const int e = t * EPT + j;
+    const uint32_t rows = e < E ? offsets[e + 1] - offsets[e] : 0u;
+    tiles[j] = tall ? (rows + (uint32_t)kTallTileRows - 1u) / (uint32_t)kTallTileRows
+                    : (rows + (uint32_t)kGemmTileRows - 1u) / (uint32_t)kGemmTileRows;  // constant divisors
+    tot += tiles[j];
+  }
+  const uint32_t s = wave_scan_u32(tot);
+  if (lane == 63) wsum[wave] = s;
+  __syncthreads();
+  uint32_t at = s - tot, all = 0;
+#pragma unroll
+  for (int w = 0; w < kPlanThreads / 64; w++) {
+    at += w < wave ? wsum[w] : 0u;
+    all += wsum[w];
+  }
+  if (blk == 0 && t == 0) items[0] = all;
+#pragma unroll
+  for (int j = 0; j < EPT; j++) {
+    const int e = t * EPT + j;
+    if (e < E) start[e] = at;
+    at += tiles[j];
+  }
+  __syncthreads();
+  for (int e = blk * (kPlanThreads / 64) + wave; e < E; e += nblk * (kPlanThreads / 64)) {
+    const uint32_t off = offsets[e], n = offsets[e + 1] - off, first = start[e];
+    for (uint32_t i = (uint32_t)lane; i * R < n; i += 64u) {
+      const uint32_t r = i * R;
+      items[4 + 2 * (first + i)] = (uint32_t)e;
+      items[5 + 2 * (first + i)] = (off + r) | ((min(n - r, R) - 1u) << shift);
+    }
+  }
 }
+// Blocks of the list: a wave per expert, up to 32 blocks.
+static int item_blocks(int E) { return std::min((E + kPlanThreads / 64 - 1) / (kPlanThreads / 64), 32); }
 
 __global__ __launch_bounds__(kPlanThreads) void gemm_items_kernel(
-    const uint32_t* __restrict__ offsets, int E, uint32_t* __restrict__ items) {
-  gemm_items_body(offsets, E, (int)blockIdx.x, items);
+    const uint32_t* __restrict__ offsets, int E, uint32_t* __restrict__ items, bool tall) {
+  gemm_items_body(offsets, E, (int)blockIdx.x, (int)gridDim.x, tall, items);
 }
 
 // Multi-block pass 3 with the grouped GEMM's row tiles: each block scatters
@@ -530,13 +566,13 @@ __global__ __launch_bounds__(kPlanThreads) void gemm_items_kernel(
 __global__ __launch_bounds__(kPlanThreads) void plan_scatter_items_kernel(
     const uint32_t* __restrict__ idx, int M, int E, const uint32_t* __restrict__ hist,
     uint32_t* perm, uint32_t* inv, const uint32_t* __restrict__ offsets,
-    uint32_t* __restrict__ items) {
+    uint32_t* __restrict__ items, bool tall) {
   __shared__ uint32_t cursor[kPlanMaxE];
   constexpr int PER = kChunk / kPlanThreads;
   const int tid = threadIdx.x, c = blockIdx.x;
   const int nchunks = (M + kChunk - 1) / kChunk;
   if (c >= nchunks) {  // block-uniform, before any barrier
-    gemm_items_body(offsets, E, c - nchunks, items);
+    gemm_items_body(offsets, E, c - nchunks, (int)gridDim.x - nchunks, tall, items);
     return;
   }
   const int begin = c * kChunk, end = min(M, begin + kChunk);
@@ -554,11 +590,12 @@ __global__ __launch_bounds__(kPlanThreads) void plan_scatter_items_kernel(
 hipError_t launch_dispatch_plan(const uint32_t* idx, int T, int k, int E, uint32_t* counts,
                                 uint32_t* offsets, uint32_t* perm, uint32_t* inv_perm,
                                 uint32_t* used, void* scratch, size_t scratch_bytes,
-                                hipStream_t st, uint32_t* items, bool* items_done) {
+                                hipStream_t st, uint32_t* items, bool tall, bool* items_done) {
   if (items_done) *items_done = false;
   const int M = T * k;
   if (E > kPlanMaxE) return hipErrorInvalidValue;
   if (plan_by_experts(M, E)) {
+    if (tall) items = nullptr;  // a list without empty slots (launch_gemm_items)
 #define MOE_PE(QUADS)                                                                              \
   hipLaunchKernelGGL((plan_experts_kernel<QUADS>), dim3(E), dim3(1024), 0, st, idx, M, E, counts,   \
                      offsets, perm, inv_perm, items ? nullptr : used, items)
@@ -583,7 +620,7 @@ hipError_t launch_dispatch_plan(const uint32_t* idx, int T, int k, int E, uint32
                      counts, offsets, used);
   if (items) {
     hipLaunchKernelGGL(plan_scatter_items_kernel, dim3(nchunks + item_blocks(E)), dim3(kPlanThreads), 0, st, idx,
-                       M, E, hist, perm, inv_perm, offsets, items);
+                       M, E, hist, perm, inv_perm, offsets, items, tall);
     if (items_done) *items_done = true;
   } else {
     hipLaunchKernelGGL(plan_scatter_kernel, dim3(nchunks), dim3(kPlanThreads), 0, st, idx, M, E,
@@ -592,9 +629,9 @@ hipError_t launch_dispatch_plan(const uint32_t* idx, int T, int k, int E, uint32
   return hipGetLastError();
 }
 
-hipError_t launch_gemm_items(const uint32_t* offsets, int E, uint32_t* items, hipStream_t st) {
+hipError_t launch_gemm_items(const uint32_t* offsets, int E, uint32_t* items, bool tall, hipStream_t st) {
   if (E > kPlanMaxE) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(gemm_items_kernel, dim3(item_blocks(E)), dim3(kPlanThreads), 0, st, offsets, E, items);
+  hipLaunchKernelGGL(gemm_items_kernel, dim3(item_blocks(E)), dim3(kPlanThreads), 0, st, offsets, E, items, tall);
   return hipGetLastError();
 }
 

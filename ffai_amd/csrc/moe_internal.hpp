@@ -192,12 +192,12 @@ hipError_t launch_route_plan(const void* logits, int dt, int T, int E, int k, co
                              uint32_t* idx, float* w, uint32_t* counts, uint32_t* offsets,
                              uint32_t* perm, uint32_t* inv, uint32_t* used, hipStream_t st);
 // With `items`, a multi-block plan also writes the GEMM's row tiles there
-// (then *items_done is set; a one-workgroup plan leaves them to
-// launch_gemm_items).
+// (then *items_done is set; a one-workgroup plan, and a block-per-expert one for
+// tall tiles, leaves them to launch_gemm_items).
 hipError_t launch_dispatch_plan(const uint32_t* idx, int T, int k, int E, uint32_t* counts,
                                 uint32_t* offsets, uint32_t* perm, uint32_t* inv_perm,
                                 uint32_t* used, void* scratch, size_t scratch_bytes,
-                                hipStream_t st, uint32_t* items = nullptr,
+                                hipStream_t st, uint32_t* items = nullptr, bool tall = false,
                                 bool* items_done = nullptr);
 size_t dispatch_scratch_bytes(int T, int k, int E);
 // Fills offsets {0, M}, used {1, 0} for a single-expert identity plan.
@@ -247,9 +247,9 @@ struct GemmArgs {
   int x_rows;
   const uint32_t* perm;      // nullable: row(p) = perm[p] / topk, else p
   int topk;
-  const uint32_t* offsets;   // [E+1] CSR over sorted positions
   const uint32_t* items;     // row tiles (launch_gemm_items)
-  int col_blocks;            // gemm_col_blocks(N, pair)
+  int tall;                  // the tall kernel, and its tiles in items
+  int col_blocks;            // gemm_col_blocks(N, pair, tall)
   void* out;                 // [M, N]
   int N, K, gsh;
   int sb_bf16;               // scales / biases stored as bf16 (else f16)
@@ -259,23 +259,27 @@ struct GemmArgs {
   float alpha, limit;
 };
 // A block takes a tile of up to kGemmTileRows of an expert's rows and
-// kGemmTileWRows weight rows (half gate, half up rows for a pair).
-constexpr int kGemmTileRows = 96;
-constexpr int kGemmTileWRows = 128;
+// kGemmTileWRows weight rows (half gate, half up rows for a pair); the tall
+// kernel up to kTallTileRows rows and kTallTileWRows weight rows.
+constexpr int kGemmTileRows = 96, kTallTileRows = 256;
+constexpr int kGemmTileWRows = 128, kTallTileWRows = 256;
 // Column blocks per row tile.
-inline int gemm_col_blocks(int N, bool gateup) {
-  const int cols = gateup ? kGemmTileWRows / 2 : kGemmTileWRows;
+inline int gemm_col_blocks(int N, bool gateup, bool tall) {
+  const int cols = (tall ? kTallTileWRows : kGemmTileWRows) / (gateup ? 2 : 1);
   return (N + cols - 1) / cols;
 }
 // Upper bound on the row tiles of a plan of M rows over E experts.
-inline long gemm_max_tiles(int M, int E) { return M / kGemmTileRows + (long)E; }
-inline size_t gemm_items_bytes(int M, int E) { return (size_t)(4 + 2 * gemm_max_tiles(M, E)) * 4; }
+inline long gemm_max_tiles(int M, int E, bool tall) {
+  return M / (tall ? kTallTileRows : kGemmTileRows) + (long)E;
+}
+inline size_t gemm_items_bytes(int M, int E) { return (size_t)(4 + 2 * gemm_max_tiles(M, E, false)) * 4; }
 // The row tiles of a plan: items[0] = slots (items[1..3] unused), then 8
 // bytes per slot: expert (kGemmNoTile: an empty slot), first sorted position |
-// (rows - 1) << 25 (at most 2^25 positions): experts ascending, an expert's
-// tiles in order.
+// (rows - 1) << kGemmRowShift (at most 2^25 positions; tall tiles: kTallRowShift,
+// at most 2^24): experts ascending, an expert's tiles in order.
+constexpr int kGemmRowShift = 25, kTallRowShift = 24;
 constexpr uint32_t kGemmNoTile = 0xFFFFFFFFu;
-hipError_t launch_gemm_items(const uint32_t* offsets, int E, uint32_t* items, hipStream_t st);
+hipError_t launch_gemm_items(const uint32_t* offsets, int E, uint32_t* items, bool tall, hipStream_t st);
 // grid: 8 * ceil(gemm_max_tiles * col_blocks / 8) blocks (the (tile, column
 // block) pairs are split evenly over the XCDs at run time; blocks without one
 // return at once).

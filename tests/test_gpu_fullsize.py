@@ -23,7 +23,8 @@ import numpy as np
 import pytest
 
 import oracle as orc
-from moe_spec import (BF16, F16, LayerSpec, cfg_gptoss, cfg_mixed, cfg_qwen3, check_close, gen_qproj,
+from moe_spec import (BF16, F16, LayerSpec, cfg_bits, cfg_gptoss, cfg_mixed, cfg_nemotron, cfg_qwen3,
+                      check_close, gen_qproj,
                       load, store, to_numpy_f32, to_torch, zipf_router_bias, ZIPF_BETA)
 
 torch = pytest.importorskip("torch")
@@ -142,6 +143,25 @@ def test_gptoss_256_gemm_path():
     dropped)."""
     info = run_full(cfg_gptoss(seed=7, expert_bias=True), 256, dict(gate_up="gemm", down="gemm"))
     assert info["hot_rows"] > 0
+
+
+def _many_rows(kind):
+    if kind == "gptoss":  # per-expert output biases, clamped SwiGLU
+        return cfg_gptoss(seed=8, n_experts=8, expert_bias=True), 2048
+    if kind == "relu2":   # one up projection, whose activation is the down GEMM's operand
+        return cfg_nemotron(seed=9, n_experts=8, hidden=2048, inter=5888, top_k=4), 2048
+    gu, dn, gs, sb, dt = kind
+    return cfg_bits(gu, dn, gs, sb, dt, seed=10, hidden=2048, inter=2880, n_experts=8, top_k=2), 4096
+
+
+@pytest.mark.parametrize("kind", ["gptoss", "relu2", (4, 4, 64, F16, BF16), (3, 6, 32, BF16, BF16),
+                                  (8, 8, 64, F16, F16), (6, 4, 64, BF16, BF16)], ids=str)
+def test_many_rows_per_expert(kind):
+    """1024 rows per expert on average and more than 700 blocks of 256 rows x
+    256 weight rows: the grouped GEMM's 256-row tiles for the gate/up pair (or
+    the single up projection) and the down projection."""
+    spec, T = _many_rows(kind)
+    run_full(spec, T, dict(gate_up="gemm", down="gemm"))
 
 
 # ------------------------------------------------- the literal float bar --

@@ -385,6 +385,46 @@ def test_expert_matmul_tile_edges(bits, dt, sb, gs, K, counts, N):
         check_close(got, ref, dt, f"tile edges bits={bits} gs={gs} K={K} rows={counts} N={N}")
 
 
+@pytest.mark.parametrize("bits,dt,sb,gs,K", [
+    (2, BF16, F16, 32, 2048), (3, F16, BF16, 64, 2112), (4, BF16, BF16, 64, 2176), (4, F16, F16, 128, 2048),
+    (5, BF16, F16, 32, 2080 + 32), (6, BF16, BF16, 64, 2112), (8, F16, F16, 64, 2048), (8, BF16, BF16, 32, 2176),
+])
+@pytest.mark.parametrize("counts,N", [((2305, 130, 3100), 7688), ((2404, 64, 2944), 7680)])
+def test_expert_matmul_tall_tiles(bits, dt, sb, gs, K, counts, N):
+    """The grouped GEMM's 256-row tiles (some 1800 rows per expert, over 700
+    blocks): last tiles of 1, 28, 64, 100 and 130 rows, a last column block of
+    8 columns, 32 to 34 chunks of K. The oracle runs on the rows at tile edges
+    and on sampled columns. Tolerance: the layer bar."""
+    from moe_spec import gen_qproj
+    rng = np.random.default_rng(bits * 10 + K + N)
+    E, M = len(counts), int(sum(counts))
+    f = 15.0 / (2 ** bits - 1)
+    p = gen_qproj(rng, E, N, K, bits, gs, sb, s_range=(0.005 * f, 0.02 * f))
+    experts = np.repeat(np.arange(E), counts).astype(np.uint32)
+    offsets = np.concatenate([[0], np.cumsum(counts)]).astype(np.int64)
+    a = store(rng.normal(0, 1, (M, K)), dt)
+    lib = _lib.load()
+    q = _lib.QProj(0, 0, 0, None, bits, gs, sb, N, K, E)
+    wt, st, bt = to_torch(p.weight.view(np.int32)), to_torch(p.scales), to_torch(p.biases)
+    q.weight, q.scales, q.biases = wt.data_ptr(), st.data_ptr(), bt.data_ptr()
+    at = to_torch(a)
+    out = torch.full((M, N), float("nan"), dtype=at.dtype, device="cuda")
+    wsb = lib.moe_expert_matmul_workspace_bytes(C.byref(q), dt, M)
+    ws = torch.empty(wsb, dtype=torch.uint8, device="cuda")
+    offt = to_torch(offsets.astype(np.int32))
+    check(lib.moe_expert_matmul(C.byref(q), _p(at), dt, None, 1, M, _p(offt), _p(out), _p(ws), wsb, _stream()))
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(out).all())  # every row and column written
+    rows = sorted({int(r) for e in range(E) for t0 in range(0, counts[e], 256)
+                   for r in (offsets[e] + t0, offsets[e] + min(t0 + 255, counts[e] - 1),
+                             offsets[e] + min(t0 + 63, counts[e] - 1), offsets[e] + min(t0 + 128, counts[e] - 1))})
+    cols = np.unique(np.concatenate([[0, 127, 128, 255, 256, N - 9, N - 8, N - 1], rng.integers(0, N, 40)]))
+    sub = orc.QProj(np.ascontiguousarray(p.weight[:, cols]), np.ascontiguousarray(p.scales[:, cols]),
+                    np.ascontiguousarray(p.biases[:, cols]), bits, gs, sb)
+    ref = orc.round_dt(orc.qgemm_rows(sub, np.ascontiguousarray(load(a, dt)[rows]), experts[rows]), dt)
+    check_close(to_numpy_f32(out)[np.ix_(rows, cols)], ref, dt, f"tall tiles bits={bits} K={K} rows={counts}")
+
+
 @pytest.mark.parametrize("counts", [(6300,), (1, 6145, 0, 0, 97, 0, 3000), (0, 0, 0, 6144)])
 def test_expert_matmul_many_tiles(counts):
     """Experts with more row tiles than a wave has lanes (64 tiles of 96 rows
