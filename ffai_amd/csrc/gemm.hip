@@ -337,8 +337,8 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& a, const GemmLds L, ui
     // A half chunk's dead units get a zero scale and bias, and zero weights in
     // the quarter at hand: the codes that follow the row, with the row's last
     // scale, could overflow f16, and infinity times a masked activation is not zero.
-    if constexpr (LAST) {
-      const uint32_t live = tail && kb >= 2 ? 0u : ~0u;
+    if (LAST && tail) {
+      const uint32_t live = kb >= 2 ? 0u : ~0u;
 #pragma unroll
       for (int j = 0; j < NT; j++)
         q.v[j] = __builtin_bit_cast(h2_t, __builtin_bit_cast(uint32_t, q.v[j]) & live);
