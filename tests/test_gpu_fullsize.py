@@ -8,7 +8,7 @@ ids, the f32 combine weights and the dispatch permutation / CSR offsets are
 bit-exact against the oracle routing from the GPU's logits, and the logits are
 within two storage ulps of the oracle's. The float output is checked against
 the fp32-accumulated oracle on a sample of tokens chosen to cover the hottest
-expert, the coldest used expert, experts whose last row tile is a half tile,
+expert, the coldest used expert, experts whose last row tile is of each height,
 tile boundaries and random tokens: a token's output depends only on its own
 input row and routing, so the oracle runs on the sampled rows with their GPU
 logits.
@@ -33,7 +33,10 @@ pytestmark = pytest.mark.gpu
 from ffai_amd import _lib  # noqa: E402
 from ffai_amd._lib import check  # noqa: E402
 
-GEMM_ROWS = 256  # rows per tile of the grouped GEMM (a half tile holds at most 128)
+# Row tiles of the grouped GEMM and the heights a last tile takes (the tall
+# kernel: 256 rows)
+GEMM_ROWS, GEMM_HEIGHTS = 96, (32, 64, 96)
+TALL_ROWS, TALL_HEIGHTS = 256, (64, 128, 256)
 
 
 @pytest.fixture(scope="module", autouse=True)
@@ -55,10 +58,11 @@ def layer_paths(dev, T):
     return p.names()
 
 
-def sample_tokens(idx, E, n_random, seed):
-    """Tokens covering the hottest and the coldest used expert, every expert
-    whose last tile is a half tile (one token each), the first and last row
-    of every tile of the hottest expert, plus random tokens."""
+def sample_tokens(idx, E, n_random, seed, rows=GEMM_ROWS, heights=GEMM_HEIGHTS):
+    """Tokens covering the hottest and the coldest used expert, the first and
+    last row of the last tile of up to 12 experts for each height that tile can
+    take, the first and last row of every tile of the hottest expert, plus random
+    tokens."""
     T, k = idx.shape
     counts = np.bincount(idx.ravel(), minlength=E)
     used = np.nonzero(counts)[0]
@@ -68,23 +72,26 @@ def sample_tokens(idx, E, n_random, seed):
     for e in (hot, cold):
         r = rows_of[e]
         pick.update(r[[0, len(r) // 2, len(r) - 1]].tolist())
-    half = [e for e in used if 0 < counts[e] % GEMM_ROWS <= GEMM_ROWS // 2]
-    for e in half:
-        r = rows_of[e]
-        last_tile0 = (len(r) - 1) // GEMM_ROWS * GEMM_ROWS
-        pick.add(int(r[last_tile0]))
-        pick.add(int(r[-1]))
+    by_height = {h: [] for h in heights}
+    for e in used:
+        last = (counts[e] - 1) % rows + 1
+        by_height[next(h for h in heights if last <= h)].append(e)
+    for es in by_height.values():
+        for e in es[:12]:
+            r = rows_of[e]
+            pick.update((int(r[(len(r) - 1) // rows * rows]), int(r[-1])))
     r = rows_of[hot]
-    for t0 in range(0, len(r), GEMM_ROWS):
+    for t0 in range(0, len(r), rows):
         pick.add(int(r[t0]))
-        pick.add(int(r[min(t0 + GEMM_ROWS, len(r)) - 1]))
+        pick.add(int(r[min(t0 + rows, len(r)) - 1]))
     rng = np.random.default_rng(seed)
     pick.update(rng.choice(T, size=n_random, replace=False).tolist())
     return np.array(sorted(pick)), dict(hot=hot, cold=cold, hot_rows=int(counts[hot]),
-                                        cold_rows=int(counts[cold]), half_tiles=len(half))
+                                        cold_rows=int(counts[cold]),
+                                        heights={h: len(es) for h, es in by_height.items()})
 
 
-def run_full(spec, T, expect, seed=0, n_random=48):
+def run_full(spec, T, expect, seed=0, n_random=48, tiles=(GEMM_ROWS, GEMM_HEIGHTS)):
     dev = spec.device()
     paths = layer_paths(dev, T)
     for key, val in expect.items():
@@ -107,7 +114,7 @@ def run_full(spec, T, expect, seed=0, n_random=48):
     assert np.array_equal(_u32(tr["perm"]), perm_ref), "dispatch permutation"
     assert np.array_equal(_u32(tr["offsets"]), off_ref), "CSR offsets"
     # float output on the sampled tokens
-    toks, info = sample_tokens(idx_ref, spec.n_experts, n_random, seed)
+    toks, info = sample_tokens(idx_ref, spec.n_experts, n_random, seed, *tiles)
     assert len(toks) >= 64, len(toks)
     y_ref, _, idx_s, _ = orc.moe_layer(spec, x[toks], given_logits=logits_gpu[toks])
     assert np.array_equal(idx_s, idx_ref[toks])
@@ -123,7 +130,7 @@ def test_prefill_4096_zipf_full_size():
     a hottest-expert load of about 10x the median."""
     spec = cfg_qwen3(seed=5, router_bias=zipf_router_bias(128, 1.1, beta=ZIPF_BETA))
     info = run_full(spec, 4096, dict(gate_up="gemm", down="gemm"))
-    assert info["half_tiles"] > 0
+    assert all(info["heights"].values()), info
 
 
 def test_mixed_2048_shared_full_size():
@@ -161,7 +168,7 @@ def test_many_rows_per_expert(kind):
     256 weight rows: the grouped GEMM's 256-row tiles for the gate/up pair (or
     the single up projection) and the down projection."""
     spec, T = _many_rows(kind)
-    run_full(spec, T, dict(gate_up="gemm", down="gemm"))
+    run_full(spec, T, dict(gate_up="gemm", down="gemm"), tiles=(TALL_ROWS, TALL_HEIGHTS))
 
 
 # ------------------------------------------------- the literal float bar --
@@ -209,8 +216,8 @@ def literal_bar(got, ref, label):
     (64, "gemv_mma", 256, 8, (3, 6)),
     (1024, "gemm", 32, 4, (4, 4)),       # grouped GEMM, 128 rows per expert
     (1024, "gemm", 32, 4, (3, 6)),
-    (256, "gemm", 16, 4, (4, 4)),        # 64 rows per expert: the 64-row tile shape
-    (320, "gemm", 16, 4, (3, 6)),        # 80 rows per expert: the 128-row tile shape
+    (256, "gemm", 16, 4, (4, 4)),        # 64 rows per expert: 64- and 96-row tiles
+    (320, "gemm", 16, 4, (3, 6)),        # 80 rows per expert
 ])
 def test_literal_tolerance_centred(T, path, E, k, bits):
     spec = cfg_centred(seed=T + E, E=E, H=2048, I=768, k=k, bits_gu=bits[0], bits_d=bits[1])

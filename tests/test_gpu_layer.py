@@ -140,10 +140,11 @@ def test_router_logits_within_one_ulp(dt, wdt, E, H, T):
     (64, 64, 2880, 64, BF16, True),    # 16 waves of 3 or 2 chunks
     (33, 65, 3072, 64, F16, False),    # 16 waves of 3 chunks
     (32, 32, 1088, 64, BF16, False),   # 16 waves of 2 or 1
-    # 256 tiles: 4 waves per tile (no bias: the bound is two ulps of the logit
-    # itself, and among 2^18 logits a bias cancels some product of magnitude 2 to
-    # 4, whose own f16 ulp is 2^-9 to 2^-8, down to a far smaller logit)
+    # 256 tiles: 4 waves per tile
     (2048, 128, 192, 32, F16, False),
+    (2048, 128, 192, 32, F16, True),
+    (2048, 128, 1024, 64, BF16, True),  # 4 waves of 4 chunks
+    (2048, 128, 1088, 64, F16, True),   # 5, 4, 4 and 4
 ])
 def test_router_logits_q(bits, T, E, H, gs, dt, bias):
     """moe_router_logits_q (an mlx QuantizedLinear router) against the oracle's
@@ -164,7 +165,11 @@ def test_router_logits_q(bits, T, E, H, gs, dt, bias):
                                           None if bt is None else _p(bt), E, _p(out), _stream()))
     torch.cuda.synchronize()
     got = to_numpy_f32(out)
-    ulp = np.abs(ref) * (2.0 ** -7 if dt == BF16 else 2.0 ** -10) + 1e-6
+    # One ulp of the rounded product and one of the rounded sum with the bias: two
+    # of the larger. (A bias can cancel a product down to a far smaller logit, whose
+    # own ulp says nothing about the product's rounding.)
+    top = np.abs(ref) if b is None else np.maximum(np.abs(ref), np.abs(orc.router_logits_q(x, dt, q, None)))
+    ulp = top * (2.0 ** -7 if dt == BF16 else 2.0 ** -10) + 1e-6
     tol = 2.02 * ulp + 1e-4 * (1.0 + np.abs(ref).max(axis=1, keepdims=True))
     assert np.all(np.abs(got - ref) <= tol), float(np.abs(got - ref).max())
     # most logits round to the oracle's value exactly (f16 rows carry three
@@ -937,15 +942,52 @@ def test_layer_mfma_path(case):
                                   (5, 2, 64, BF16, F16)],
                          ids=lambda c: f"gu{c[0]}-d{c[1]}-gs{c[2]}-sb{c[3]}-x{c[4]}")
 def test_layer_batched_mma_path(case):
-    """Up to 23 rows per used expert on average with 2- to 6-bit weights (24
-    and more take the grouped GEMM): the batched GEMV on
-    the matrix cores (codes of 3, 5 and 6 bits straddle words inside a lane's
-    8-value block), with a partial last block of down rows (hidden 544 is 8.5
-    blocks of 64) and passes of 16 activation rows (up to 30 rows for one
-    expert at T = 40, 8 experts, top-3)."""
+    """15 rows per used expert on average with 2- to 6-bit weights (24 and more
+    take the grouped GEMM): the batched GEMV on the matrix cores (codes of 3, 5
+    and 6 bits straddle words inside a lane's 8-value block), with a partial last
+    block of down rows (hidden 544 is 8.5 blocks of 64); 4-bit projections run
+    passes of 32 activation rows, the others of 16 (up to 30 rows for one expert
+    at T = 40, 8 experts, top-3)."""
     gs = case[2]
     hidden = 544 if gs == 32 else 640
     run_layer(cfg_bits(*case, hidden=hidden, inter=384, n_experts=8, top_k=3), 40)
+
+
+def _paths(dev, T):
+    p = _lib.LayerPaths()
+    check(_lib.load().moe_layer_path(C.byref(dev.desc), T, C.byref(p)))
+    return p.names()
+
+
+@pytest.mark.parametrize("T,hot", [
+    (14, False),  # 5 rows per expert on average: passes of 16 rows
+    (45, False),  # 17: of 32 at 4 and 8 bits
+    (38, True),   # 14 on average, one expert with every row: three passes of 16
+    (56, True),   # 21 on average, two passes of 32
+])
+@pytest.mark.parametrize("case", [(8, 8, 32, F16, F16), (8, 8, 64, BF16, BF16), (8, 4, 128, BF16, F16),
+                                  (4, 8, 64, F16, BF16), (4, 4, 32, BF16, BF16)],
+                         ids=lambda c: f"gu{c[0]}-d{c[1]}-gs{c[2]}-sb{c[3]}-x{c[4]}")
+def test_layer_mma_pair_passes(case, T, hot):
+    """Gate/up pairs on the matrix-core GEMV at 4 and 8 bits: one and several
+    passes of 16 and of 32 activation rows (a pass's gate outputs take the place
+    of an activation stage that the next pass fills again)."""
+    spec = cfg_bits(*case, hidden=640, inter=384, n_experts=8, top_k=3)
+    if hot:
+        spec.router_bias = store(np.where(np.arange(8) == 5, 8.0, 0.0), spec.act_dt)
+    dev, x, _ = run_layer(spec, T, seed=T)
+    paths = _paths(dev, T)
+    assert (paths["gate_up"], paths["down"]) == ("gemv_mma", "gemv_mma")
+    if hot:
+        idx, _ = orc.route(spec.oracle_logits(x), 3, spec.gating, spec.norm_topk)
+        assert (idx == 5).sum() == T
+
+
+def test_layer_used_list_past_512_entries(mixed):
+    """100 tokens x top-8 on 256 experts: 800 entries, planned by a block per
+    expert, whose used list the matrix-core GEMV takes its experts from."""
+    dev, _, _ = run_layer(mixed, 100, seed=6)
+    assert _paths(dev, 100)["gate_up"] == "gemv_mma"
 
 
 def test_layer_qwen3_mfma_zipf():
