@@ -480,9 +480,9 @@ struct Workspace {
 };
 
 // Bytes a workspace holds for the GEMM's list over N outputs: 16 per 256-row
-// tile and 128 (gate/up) or 256 columns, more than two such regions' tile list
-// needs (8 bytes per 96-row tile: M / 12 + 8 E against M / 8 + 32 E at one
-// column block each). The size stays what it was with one item per column
+// tile and 128 (gate/up) or 256 columns, more in two such regions than the tile
+// list needs (8 bytes per 96- or 256-row tile: M / 12 + 8 E against M / 8 + 32 E at
+// one column block each). The size stays what it was with one item per column
 // block, so that a workspace size, and which calls fit the allocation-free
 // entry's fixed one, does not depend on the tiling.
 size_t gemm_list_bytes(size_t M, size_t E, size_t N, bool gateup) {
@@ -552,7 +552,11 @@ constexpr int kMultiBlocks = 512;
 // (Qwen3 shape, 4 per expert: 192 -> 154 us per layer step; GPT-OSS, 8 per
 // expert: 409 -> 208 us; at 1 per expert gemv_multi_kernel is faster).
 // Codes of other widths cost gemv_multi_kernel more unpacking, so they move
-// from 2 rows per expert (mixed 3/6-bit layer, 64 tokens: 317 -> 231 us).
+// from 2 rows per expert (mixed 3/6-bit layer, 64 tokens: 317 -> 231 us; 8 bits,
+// gemv_multi_kernel / here: 64 experts of 1024 x 384, 2 rows 61.2 / 41.6, 128
+// experts of 2048 x 768, 2 rows 194 / 133, 32 of 2880 x 2880, 2 rows 323 / 222; f16
+// with groups of 32 there 234 / 239, 3 rows 310 / 270; below 2 rows gemv_multi_kernel
+// was not compared).
 // One expert alone (a shared expert) gets only ceil(N / 32) matrix-core
 // blocks, so it moves only once a pass fills the 16 activation rows.
 // 4-bit thresholds re-measured after the matrix-core GEMV's loop and
@@ -680,9 +684,9 @@ void run_multi(const moe_qproj& p0, const moe_qproj* p1, const void* x, int xdt,
   *status = hip_check(err, "grouped GEMV launch");
 }
 
-// gemv_mma_kernel (matrix cores) for 16-bit
-// activations: 32 rows of a gate/up pair or 64 rows of one projection per
-// block, 16 activation rows per pass. The caller has checked mma_ok.
+// gemv_mma_kernel (matrix cores) for 16-bit activations: 32 rows of a gate/up
+// pair or 64 rows of one projection per block, 16 or 32 activation rows per pass.
+// The caller has checked mma_ok.
 void run_mma(const moe_qproj& p0, const moe_qproj* p1, const void* x, int xdt,
              const uint32_t* perm, int topk, const uint32_t* offsets, const uint32_t* used, int slots,
              int M, int max_rows, int x_rows, void* out, int act, float alpha, float limit, hipStream_t st,
@@ -760,9 +764,11 @@ moe_status run_gemv(const moe_qproj& p0, const moe_qproj* p1, const void* x, int
   return MOE_OK;
 }
 
-// The MFMA grouped GEMM pays off once the used experts average enough rows
-// to fill a good part of its 64-row tiles; below that the matrix-core GEMV,
-// which reads every weight once per 16 rows, is faster. Swept at 16 / 24 /
+// The MFMA grouped GEMM pays off once the used experts average enough rows to
+// share its dequantised weights; below that the matrix-core GEMV, which reads
+// every weight once per 16 or 32 rows, is faster. Swept with the GEMM's tiles of
+// 64 to 256 rows and the GEMV's passes of 16, before either's present form (the
+// lines have not been swept again since), at 16 / 24 /
 // 32+ rows per expert (µs per layer step, GEMV against GEMM): 16 rows
 // Qwen3 192.8 / 184.4, GPT-OSS 254.0 / 301.9, mixed-bit 317.3 / 320.0; 24
 // rows Qwen3 242.0 / 191.8, GPT-OSS 323.9 / 305.3, mixed-bit 381.2 / 321.1.

@@ -47,10 +47,9 @@
 // with the weights through LDS (us per layer step): 2048 tokens on 256 3/6-bit
 // experts 347 -> 289 (gate/up launch 189 -> 153, down 119 -> 99), 1000 tokens
 // on 32 experts of 2880 x 2880 at 4 bits 393 -> 358, 4096 tokens on 128 experts
-// with Zipf loads 460-494 -> 461-478 by box and run: there the two GEMM launches
-// are 5 % longer (302 + 175 us, was 293 + 161: most tiles are full, and taller
-// ones share a weight fetch better) and the shorter plan and router launches
-// make up for it.
+// with Zipf loads 460-494 -> 461-478 by box and run (gate/up launch 270 -> 261,
+// down 150 -> 154). From some hundreds of rows per expert on, tall tiles share a
+// weight fetch better: gemm_tall.hip (gemm_tall in api.cpp has the line).
 // Storing the tile through LDS, whole row segments at a time, changed nothing
 // (470 / 286 / 357 us against 470 / 288 / 355 for the last, first and second case).
 // Not kept: 256 weight rows per block (four 16-row tiles per wave, 2 waves per

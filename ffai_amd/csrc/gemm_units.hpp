@@ -68,7 +68,7 @@ __device__ __forceinline__ void quarter_pairs(const uint32_t (&w)[BITS], int s, 
       pr[2 * h] = (m & kPair) | M;
       pr[2 * h + 1] = ((m >> (2 * BITS)) & kPair) | M;
     }
-  } else if constexpr (BITS == 5 || BITS == 6) {
+  } else {  // 5 and 6 bits
     // A pair's 2 * BITS bits lie inside the 16 bits from the byte holding its
     // first bit: one byte permute puts those 16 bits in both halves, and one
     // packed 16-bit shift right by (o, o + BITS) brings each value to the
@@ -84,19 +84,6 @@ __device__ __forceinline__ void quarter_pairs(const uint32_t (&w)[BITS], int s, 
       const u16x2_t z = __builtin_bit_cast(u16x2_t, __builtin_amdgcn_perm(w[wj], w[wi], sel));
       const u16x2_t t = z >> u16x2_t{(unsigned short)o, (unsigned short)(o + BITS)};
       pr[p] = (__builtin_bit_cast(uint32_t, t) & kPair) | M;
-    }
-  } else {
-#pragma unroll
-    for (int p = 0; p < 4; p++) {
-      uint32_t c[2];
-#pragma unroll
-      for (int k = 0; k < 2; k++) {
-        const int bit = (8 * s + 2 * p + k) * BITS, lo = bit >> 5, sh = bit & 31;
-        uint32_t v = w[lo] >> sh;
-        if (sh + BITS > 32) v |= w[lo + 1] << (32 - sh);
-        c[k] = v & ((1u << BITS) - 1u);
-      }
-      pr[p] = (c[0] | (c[1] << 16)) | M;
     }
   }
 }

@@ -428,8 +428,9 @@ template <> struct Mma16<f16_t> {
   }
 };
 
-// Units per K chunk: a 128-byte line of a weight row at 4 and 8 bits (half the
-// LDS per 8-bit chunk keeps five blocks per CU instead of two).
+// Units per K chunk: a 128-byte line of a weight row at 4 and 8 bits (the LDS of
+// eight 8-bit units, 53 KB, would hold three blocks per CU, where the registers
+// allow four).
 template <int BITS> constexpr int kMmaUnits = BITS == 8 ? 4 : 8;
 constexpr int kMmaRows = 64;  // LDS weight rows per block
 
