@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """MoE-layer benchmark on one MI355X.
 
-Default workload: BASELINE.json configs[1], a GPT-OSS-20B-shaped MoE decode
+Default workload: a GPT-OSS-20B-shaped MoE decode
 layer (hidden = intermediate = 2880, 32 experts, top-4 on logits then softmax,
 clamped SwiGLU, mlx affine 4-bit gs64 with bf16 scales/biases, biased bf16
 router) on one token. 24 independent layers' weights stay resident in HBM
@@ -18,11 +18,11 @@ Prints one JSON line:
               hipEvents on the launch stream; `rocprof` beside it divides the
               same bytes by the committed rocprofv3 average of that kernel
   cpu_baseline the C oracle (oracle/) on layer 0, one token at a time
-The default line also carries configs[3] (`prefill`), configs[4] (`mixed`),
-configs[4]'s layer at one token (`mixed1`) and the configs[2] sweep
-(`qwen3_decode`, 1 / 4 / 16 / 64 tokens).
-Other configs: --config qwen3 (configs[2], --batch B), prefill,
-mixed; --config ckpt_load times the checkpoint reader loading
+The default line also carries the Qwen3-MoE-shaped prefill of 4096 tokens
+(`prefill`), the mixed 3/6-bit one of 2048 (`mixed`), that layer at one token
+(`mixed1`) and the Qwen3-MoE-shaped decode sweep (`qwen3_decode`, 1 / 4 / 16 / 64
+tokens).
+Other configs: --config qwen3 (--batch B), prefill, mixed; --config ckpt_load times the checkpoint reader loading
 stacked mlx-affine experts from the page cache into HBM.
 """
 from __future__ import annotations
@@ -56,7 +56,7 @@ CONFIGS = {
     "mixed": dict(H=2048, E=256, k=8, I=512, bits_gu=3, bits_d=6, sb="bf16", act="swiglu",
                   gating="softmax_topk", router_bias=False, T=2048, SI=512,
                   workload="mixed_3b6b_shared_prefill_2048"),
-    # configs[4]'s layer at one token: the 3/6-bit one-token kernels
+    # the mixed layer at one token: the 3/6-bit one-token kernels
     "mixed1": dict(H=2048, E=256, k=8, I=512, bits_gu=3, bits_d=6, sb="bf16", act="swiglu",
                    gating="softmax_topk", router_bias=False, T=1, SI=512,
                    workload="mixed_3b6b_shared_decode_b1"),
@@ -626,9 +626,8 @@ def main():
         "expert_stream": res["expert_stream"],
     }
     if args.config == "gptoss" and not args.batch and not args.no_extra:
-        # the metric's other two parts, on the prefill configs (configs[3],
-        # configs[4]): fixed counts, independent of --steps / --warmup
-        # plus the one-token 3/6-bit row (configs[4]'s layer at T = 1)
+        # the metric's other two parts, on the two prefills: fixed counts,
+        # independent of --steps / --warmup, plus the one-token 3/6-bit row
         for name, st2, wu2, L2 in (("prefill", 60, 6, 4), ("mixed", 60, 6, 4), ("mixed1", 480, 48, 24)):
             c2 = dict(CONFIGS[name])
             r2, _ = run_config(c2, torch, fl, lib, steps=st2, warmup=wu2, L=L2)
@@ -640,7 +639,7 @@ def main():
                          "timed_layers": r2["config"]["timed_layers"]}
             if "zipf" in r2["config"]:
                 out[name]["zipf"] = r2["config"]["zipf"]
-        # configs[2]: the Qwen3-MoE-shaped decode sweep over batch sizes, on
+        # the Qwen3-MoE-shaped decode sweep over batch sizes, on
         # one set of 24 resident layers (8.2 GB)
         qcfg = dict(CONFIGS["qwen3"])
         qlayers = build_layers(qcfg, args.layers, torch, fl, lib)

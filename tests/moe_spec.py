@@ -1,4 +1,4 @@
-"""Synthetic MoE layers for the parity tests (BASELINE.json configs) and the
+"""Synthetic MoE layers for the parity tests and the
 glue that hands the same numpy arrays to the CPU oracle and to libmoehip.so.
 """
 from __future__ import annotations
@@ -210,7 +210,7 @@ def to_numpy_f32(t):
 # ---------------------------------------------------------------- configs --
 
 def cfg_tiny(seed=0, act_dt=F16):
-    """configs[0]: hidden=256, 8 experts, top-2, I=512, 4-bit gs64, f16."""
+    """hidden=256, 8 experts, top-2, I=512, 4-bit gs64, f16."""
     rng = np.random.default_rng(seed)
     H, E, k, I = 256, 8, 2, 512
     return LayerSpec(H, E, k, I, act_dt,
@@ -220,7 +220,7 @@ def cfg_tiny(seed=0, act_dt=F16):
 
 
 def cfg_gptoss(seed=0, n_experts=32, hidden=2880, inter=2880, expert_bias=False):
-    """configs[1]: GPT-OSS-20B-shaped decode layer (4-bit gs64, bf16)."""
+    """GPT-OSS-20B-shaped decode layer (4-bit gs64, bf16)."""
     rng = np.random.default_rng(seed)
     H, E, k, I = hidden, n_experts, 4, inter
     ob = BF16 if expert_bias else None
@@ -235,7 +235,7 @@ def cfg_gptoss(seed=0, n_experts=32, hidden=2880, inter=2880, expert_bias=False)
 
 
 def cfg_qwen3(seed=0, n_experts=128, hidden=2048, inter=768, router_bias=None):
-    """configs[2]/[3]: Qwen3-MoE shape, 4-bit gs64, fp16 scales, bf16 acts."""
+    """Qwen3-MoE shape, 4-bit gs64, fp16 scales, bf16 acts."""
     rng = np.random.default_rng(seed)
     H, E, k, I = hidden, n_experts, 8, inter
     return LayerSpec(H, E, k, I, BF16,
@@ -246,7 +246,7 @@ def cfg_qwen3(seed=0, n_experts=128, hidden=2048, inter=768, router_bias=None):
                      down=gen_qproj(rng, E, H, I, 4, 64, F16), name="qwen3")
 
 
-# Router-bias strength for configs[3]: beta * log p with p Zipf(1.1) gives a
+# Router-bias strength for the 4096-token prefill: beta * log p with p Zipf(1.1) gives a
 # hottest-expert load of about 10x the median at 0.33 (4096 tokens, 128
 # experts, top-8: max / median 9.9-10.0 over two seeds; beta = 1.0 gives
 # about 230x, nearly every token on the hottest expert).
@@ -263,7 +263,7 @@ def zipf_router_bias(E, s=1.1, beta=ZIPF_BETA, seed=0):
 
 
 def cfg_mixed(seed=0, n_experts=256, hidden=2048, inter=512, shared_inter=512):
-    """configs[4]: 3-bit gate/up, 6-bit down, bf16 scales, shared expert with
+    """3-bit gate/up, 6-bit down, bf16 scales, shared expert with
     a sigmoid gate."""
     rng = np.random.default_rng(seed)
     H, E, k, I = hidden, n_experts, 8, inter

@@ -1,7 +1,7 @@
 """Parity at the benchmarked prefill sizes, on the kernels those sizes run.
 
-configs[3] (Qwen3-MoE-shaped, 4096 tokens, 128 experts, Zipf(1.1) router
-skew) and configs[4] (2048 tokens, 256 experts, 3-bit gate/up, 6-bit down,
+A Qwen3-MoE-shaped layer (4096 tokens, 128 experts, Zipf(1.1) router skew)
+and a mixed-width one (2048 tokens, 256 experts, 3-bit gate/up, 6-bit down,
 sigmoid-gated shared expert) go through the grouped GEMM on the matrix cores;
 each test first asserts that path (moe_layer_path). For every token the expert
 ids, the f32 combine weights and the dispatch permutation / CSR offsets are
@@ -13,7 +13,7 @@ tile boundaries and random tokens: a token's output depends only on its own
 input row and routing, so the oracle runs on the sampled rows with their GPU
 logits.
 
-The literal north-star bar, max |d| <= 2e-2 and mean |d| / mean |ref| <= 1e-3
+The literal bar, max |d| <= 2e-2 and mean |d| / mean |ref| <= 1e-3
 with no rescaling, is asserted on layers whose weights are centred the way
 mlx checkpoints are (bias about -scale * (2^bits - 1) / 2), so outputs are
 O(1), on the one-token, batched matrix-core GEMV and grouped-GEMM paths."""
@@ -126,7 +126,7 @@ def run_full(spec, T, expect, seed=0, n_random=48, tiles=(GEMM_ROWS, GEMM_HEIGHT
 
 
 def test_prefill_4096_zipf_full_size():
-    """configs[3]: 4096 tokens, 128 experts, top-8, Zipf(1.1) skew calibrated to
+    """4096 tokens, 128 experts, top-8, Zipf(1.1) skew calibrated to
     a hottest-expert load of about 10x the median."""
     spec = cfg_qwen3(seed=5, router_bias=zipf_router_bias(128, 1.1, beta=ZIPF_BETA))
     info = run_full(spec, 4096, dict(gate_up="gemm", down="gemm"))
@@ -134,7 +134,7 @@ def test_prefill_4096_zipf_full_size():
 
 
 def test_mixed_2048_shared_full_size():
-    """configs[4]: 2048 tokens, 256 experts, 3-bit gate/up and 6-bit down, and
+    """2048 tokens, 256 experts, 3-bit gate/up and 6-bit down, and
     the sigmoid-gated shared expert on its side stream."""
     info = run_full(cfg_mixed(), 2048, dict(gate_up="gemm", down="gemm", shared_gate_up="gemm",
                                             shared_down="gemm"))

@@ -643,7 +643,7 @@ def test_layer_given_logits_path_is_identical():
 
 
 def test_layer_tiny_matches_float64_composition():
-    """Whole tiny layer (configs[0]) against a float64 composition of
+    """Whole tiny layer against a float64 composition of
     independently dequantised experts with the same storage rounding points."""
     from moe_spec import cfg_tiny, load, store
     spec = cfg_tiny()
